@@ -489,95 +489,6 @@ __device__ __forceinline__ int64_t total_steps(const AttnParams& p, int lane) {
 // every segment between the first and last one covering a sequence holds part of it.
 __device__ __forceinline__ int64_t seg_len(int64_t S, int nseg) { return (S + nseg - 1) / nseg; }
 
-// Merge the nparts partials of (sequence b, kv-head kh), stored at slots f+b .. f+nparts-1+b,
-// into the final rows.  Thread t (of 256) handles row t / 16 and DS = D / 16 consecutive head
-// dims.  Up to KB pieces are loaded together (every load issued before any is used; indices
-// clamped into range, surplus pieces weighted zero), so a sequence of up to KB partials -- at
-// the config 3 batch every one -- costs one memory round trip.
-template <typename TT, int D>
-__device__ __forceinline__ void merge_pieces(const AttnParams& p, int b, int kh, int s0, int R,
-                                             int g, int f, int nparts, int tid) {
-  constexpr int DS = D / 16;           // dims per thread
-  constexpr int KB = D > 128 ? 6 : 96 / DS;  // pieces per batch (~96 registers of partials)
-  static_assert(DS % 2 == 0, "pairs of dims");
-  const int r = tid >> 4, slice = tid & 15;
-  if (r >= R) return;
-  float M = kNegInf, lsum = 0.0f;
-  float acc[DS];
-#pragma unroll
-  for (int e = 0; e < DS; ++e) acc[e] = 0.0f;
-  for (int k0 = 0; k0 < nparts; k0 += KB) {
-    float2 ml[KB];
-    float o[KB][DS];
-#pragma unroll
-    for (int j = 0; j < KB; ++j) {
-      const int k = min(k0 + j, nparts - 1);
-      const int64_t row = (((int64_t)f + k + b) * p.kv_heads + kh) * 16 + r;
-      ml[j] = *reinterpret_cast<const float2*>(p.part_ml + row * 2);
-      const float* src = p.part_o + row * D + slice * DS;
-      if constexpr (DS % 4 == 0) {
-#pragma unroll
-        for (int v = 0; v < DS / 4; ++v) {
-          const f32x4 x = reinterpret_cast<const f32x4*>(src)[v];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[j][4 * v + e] = x[e];
-        }
-      } else {
-#pragma unroll
-        for (int v = 0; v < DS / 2; ++v) {
-          const float2 x = reinterpret_cast<const float2*>(src)[v];
-          o[j][2 * v] = x.x;
-          o[j][2 * v + 1] = x.y;
-        }
-      }
-    }
-    float mn = M;
-#pragma unroll
-    for (int j = 0; j < KB; ++j)
-      if (k0 + j < nparts) mn = fmaxf(mn, ml[j].x);
-    // mn == -inf (every piece so far saw only masked keys) leaves a = w = 0 below.
-    const float a = (M == kNegInf) ? 0.0f : exp2f(M - mn);
-    lsum *= a;
-#pragma unroll
-    for (int e = 0; e < DS; ++e) acc[e] *= a;
-#pragma unroll
-    for (int j = 0; j < KB; ++j) {
-      const float w = (k0 + j < nparts && ml[j].x != kNegInf) ? exp2f(ml[j].x - mn) : 0.0f;
-      lsum += ml[j].y * w;
-#pragma unroll
-      for (int e = 0; e < DS; ++e) acc[e] += o[j][e] * w;
-    }
-    M = mn;
-  }
-  const int h = kh * g + r % g;
-  const int64_t t = s0 + r / g;
-  const float fct = finalize_factor(M, lsum, sink_logit<TT>(p, h));
-  if (p.v_quant == PA_QUANT_PER_TENSOR || p.v_quant == PA_QUANT_PER_CHANNEL) {
-    // integer pages: the partials are in code units; scale each output dim
-    const bool pc = p.v_quant == PA_QUANT_PER_CHANNEL;
-#pragma unroll
-    for (int e = 0; e < DS; ++e)
-      acc[e] *= pc ? p.v_scale[(int64_t)kh * D + slice * DS + e] : p.v_scale[0];
-  }
-  uint32_t w[DS / 2];
-#pragma unroll
-  for (int m = 0; m < DS / 2; ++m)
-    w[m] = (uint32_t)TT::from_f32(acc[2 * m] * fct) |
-           ((uint32_t)TT::from_f32(acc[2 * m + 1] * fct) << 16);
-  uint32_t* out = reinterpret_cast<uint32_t*>(reinterpret_cast<typename TT::raw*>(p.out) +
-                                              (t * p.num_heads + h) * D + slice * DS);
-  if constexpr (DS % 8 == 0) {
-#pragma unroll
-    for (int v = 0; v < DS / 8; ++v)
-      reinterpret_cast<u32x4*>(out)[v] = u32x4{w[4 * v], w[4 * v + 1], w[4 * v + 2], w[4 * v + 3]};
-  } else if constexpr (DS == 4) {
-    *reinterpret_cast<u32x2*>(out) = u32x2{w[0], w[1]};
-  } else {
-#pragma unroll
-    for (int m = 0; m < DS / 2; ++m) out[m] = w[m];
-  }
-}
-
 // Up to 64 consecutive sequences, lane l describing sequence base + l.
 struct SeqWin {
   int base;
@@ -1271,13 +1182,30 @@ decode_balanced_kernel(const AttnParams p) {
   }
 }
 
-// Merge the partials of every (kv-head, sequence) split across segments (one workgroup each).
+// Merge the partials of every sequence split across segments: a workgroup takes one slice of SL
+// head dims of one row of (sequence, kv-head).  LP lanes hold a partial's slice (16 bytes each) and
+// the workgroup's PG groups of lanes take partials g, g + PG, ..., kMergeDepth of them in flight
+// (indices clamped, surplus ones weighted zero), so a row of up to PG * kMergeDepth partials costs
+// one memory round trip after the metadata; the groups then meet through lane exchanges and LDS.
+// Latency-bound.  With one workgroup per (kv-head, sequence) walking all rows and dims, a lone
+// 16K-token sequence at head 256 (256 partials of 24 rows on 4 workgroups) took 114 us and now
+// 6.6; 64 sequences of up to 5 partials (32 heads, head 128) 6.5 and now 5.2; 8 short ones 7.7 and
+// now 5.0.
 // A device-scope fence per piece inside the decode kernel (to let the last piece merge) writes
 // back the XCD's L2 and measured far slower than this separate launch.
-template <typename TT, int D>
-__global__ __launch_bounds__(256) void balanced_merge_kernel(const AttnParams p) {
-  const int kh = blockIdx.x, b = blockIdx.y;
-  const int lane = threadIdx.x & 63;
+constexpr int kMergeDepth = 4;
+// Head dims of a workgroup's slice: 64 (16 lanes per partial), 32 at head 96; the one-wavefront
+// workgroups of batches with few partials per sequence take up to 256, for fewer workgroups.
+template <int D, int NT>
+constexpr int merge_slice() {
+  return D % 64 != 0 ? 32 : NT > 64 ? 64 : D;
+}
+template <typename TT, int D, int NT>
+__global__ __launch_bounds__(NT) void balanced_merge_kernel(const AttnParams p) {
+  constexpr int SL = merge_slice<D, NT>(), LP = SL / 4, PG = NT / LP, NW = NT / 64;
+  const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int kh = blockIdx.x % p.kv_heads, rest = blockIdx.x / p.kv_heads;
+  const int slice = rest % (D / SL), r = rest / (D / SL);
   const int nseg = p.max_splits;
   const int g = p.num_heads / p.kv_heads;
   // Prefix of steps up to b, b's own metadata and the total, one parallel pass over sequences.
@@ -1295,12 +1223,85 @@ __global__ __launch_bounds__(256) void balanced_merge_kernel(const AttnParams p)
     }
     S += __shfl(incl, 63, 64);
   }
-  if (nb <= 0 || S <= 0) return;
+  if (nb <= 0 || S <= 0 || r >= g * nq) return;
   const int64_t seg_l = seg_len(S, nseg);
   const int f = (int)(Pb / seg_l);
   const int nparts = (int)((Pb + nb - 1) / seg_l) - f + 1;
   if (nparts <= 1) return;  // written directly by the decode kernel
-  merge_pieces<TT, D>(p, b, kh, s0, g * nq, g, f, nparts, (int)threadIdx.x);
+
+  const int grp = tid / LP, d0 = slice * SL + 4 * (tid % LP);
+  const int64_t row0 = (((int64_t)f + b) * p.kv_heads + kh) * 16 + r;
+  const int64_t pitch = (int64_t)p.kv_heads * 16;  // rows between consecutive partials
+  float M = kNegInf, lsum = 0.0f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = grp; k0 < nparts; k0 += PG * kMergeDepth) {
+    float2 ml[kMergeDepth];
+    f32x4 o[kMergeDepth];
+#pragma unroll
+    for (int j = 0; j < kMergeDepth; ++j) {
+      const int64_t row = row0 + min(k0 + j * PG, nparts - 1) * pitch;
+      ml[j] = *reinterpret_cast<const float2*>(p.part_ml + row * 2);
+      o[j] = *reinterpret_cast<const f32x4*>(p.part_o + row * D + d0);
+    }
+    float mn = M;
+#pragma unroll
+    for (int j = 0; j < kMergeDepth; ++j)
+      if (k0 + j * PG < nparts) mn = fmaxf(mn, ml[j].x);
+    // mn == -inf (every piece so far saw only masked keys) leaves a = w = 0 below.
+    const float a = (M == kNegInf) ? 0.0f : exp2f(M - mn);
+    lsum *= a;
+    acc *= a;
+#pragma unroll
+    for (int j = 0; j < kMergeDepth; ++j) {
+      const float w = (k0 + j * PG < nparts && ml[j].x != kNegInf) ? exp2f(ml[j].x - mn) : 0.0f;
+      lsum += ml[j].y * w;
+      // a surplus piece's row may hold anything in a piece that saw no key: not multiplied in
+      if (w != 0.0f) acc += o[j] * w;
+    }
+    M = mn;
+  }
+  auto meet = [&](float m2, float l2, f32x4 a2) {
+    const float mn = fmaxf(M, m2);
+    const float wa = (M == kNegInf) ? 0.0f : exp2f(M - mn);
+    const float wb = (m2 == kNegInf) ? 0.0f : exp2f(m2 - mn);
+    lsum = lsum * wa + l2 * wb;
+    acc = acc * wa + a2 * wb;
+    M = mn;
+  };
+#pragma unroll
+  for (int o = LP; o < 64; o <<= 1) {
+    const f32x4 a2 = {__shfl_xor(acc[0], o, 64), __shfl_xor(acc[1], o, 64),
+                      __shfl_xor(acc[2], o, 64), __shfl_xor(acc[3], o, 64)};
+    meet(__shfl_xor(M, o, 64), __shfl_xor(lsum, o, 64), a2);
+  }
+  if constexpr (NW > 1) {
+    __shared__ f32x4 wacc[NW][LP];
+    __shared__ float2 wml[NW];
+    if (lane < LP) wacc[tid >> 6][lane] = acc;
+    if (lane == 0) wml[tid >> 6] = float2{M, lsum};
+    __syncthreads();
+    if (tid >= LP) return;
+#pragma unroll
+    for (int w = 1; w < NW; ++w) meet(wml[w].x, wml[w].y, wacc[w][tid]);
+  } else if (tid >= LP) {
+    return;
+  }
+  const int h = kh * g + r % g;
+  const int64_t t = s0 + r / g;
+  const float fct = finalize_factor(M, lsum, sink_logit<TT>(p, h));
+  if (p.v_quant == PA_QUANT_PER_TENSOR || p.v_quant == PA_QUANT_PER_CHANNEL) {
+    // integer pages: the partials are in code units; scale each output dim
+    const bool pc = p.v_quant == PA_QUANT_PER_CHANNEL;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] *= pc ? p.v_scale[(int64_t)kh * D + d0 + e] : p.v_scale[0];
+  }
+  u32x2 w;
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+    w[m] = (uint32_t)TT::from_f32(acc[2 * m] * fct) |
+           ((uint32_t)TT::from_f32(acc[2 * m + 1] * fct) << 16);
+  *reinterpret_cast<u32x2*>(reinterpret_cast<typename TT::raw*>(p.out) +
+                            (t * p.num_heads + h) * D + d0) = w;
 }
 
 template <typename TT, int D, bool CAP>
@@ -1405,15 +1406,33 @@ hipError_t launch_decode_mfma(const AttnParams& p, pa_dtype act, pa_dtype cache_
   return launch_t<TBF16>(p, grid, dim3(64), false, kDcT, s);
 }
 
-// The partial merge of the balanced decode, for the head size of the decode launch.
+// The partial merge of the balanced decode, for the head size of the decode launch.  Threads per
+// workgroup by the partials an average sequence has (max_splits / batch): 64 hold 4 groups of 4
+// partials in flight, 256 four times and 1024 sixteen times as many, all of an average row in one
+// round trip; more threads than that only wait on each other.
+template <typename TT, int D, int NT>
+void launch_merge_nt(const AttnParams& p, hipStream_t s) {
+  const int rows = std::min(16, (p.num_heads / p.kv_heads) * std::max(p.max_query_len, 1));
+  const dim3 grid(p.kv_heads * (D / merge_slice<D, NT>()) * rows, p.batch);
+  hipLaunchKernelGGL((balanced_merge_kernel<TT, D, NT>), grid, dim3(NT), 0, s, p);
+}
+template <typename TT, int D>
+void launch_merge_d(const AttnParams& p, hipStream_t s) {
+  const int parts = p.max_splits / std::max(p.batch, 1);
+  if (parts <= 8)
+    launch_merge_nt<TT, D, 64>(p, s);
+  else if (parts <= 64)
+    launch_merge_nt<TT, D, 256>(p, s);
+  else
+    launch_merge_nt<TT, D, 1024>(p, s);
+}
 template <typename TT>
 hipError_t launch_merge(const AttnParams& p, hipStream_t s) {
-  const dim3 grid(p.kv_heads, p.batch), block(256);
   switch (p.head_dim) {
-    case 64: hipLaunchKernelGGL((balanced_merge_kernel<TT, 64>), grid, block, 0, s, p); break;
-    case 96: hipLaunchKernelGGL((balanced_merge_kernel<TT, 96>), grid, block, 0, s, p); break;
-    case 128: hipLaunchKernelGGL((balanced_merge_kernel<TT, 128>), grid, block, 0, s, p); break;
-    case 256: hipLaunchKernelGGL((balanced_merge_kernel<TT, 256>), grid, block, 0, s, p); break;
+    case 64: launch_merge_d<TT, 64>(p, s); break;
+    case 96: launch_merge_d<TT, 96>(p, s); break;
+    case 128: launch_merge_d<TT, 128>(p, s); break;
+    case 256: launch_merge_d<TT, 256>(p, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
