@@ -13,6 +13,8 @@
 // Integer caches (int8, int4 nibble pairs) store sat(RNE(x / scale)) codes of the final T row
 // (QuantizedCache::encode, kv_cache.rs:170-219).
 
+#include <algorithm>
+
 #include "pa_device.hpp"
 
 #pragma clang fp contract(off)
@@ -30,6 +32,15 @@ __device__ __forceinline__ float rot_sub32(float a, float c, float b, float s) {
 __device__ __forceinline__ float rot_add32(float a, float c, float b, float s) {
   const float x = a * c, y = b * s;
   return x + y;
+}
+
+// a * b rounded to fp32 before anything else rounds it: without the barrier the compiler joins the
+// product of a norm and its rounding to fp16 into one v_fma_mixlo_f16 here and there, whose single
+// rounding differs from the two of the reference's graph about once in 25,000 elements.
+__device__ __forceinline__ float mul32(float a, float b) {
+  float x = a * b;
+  asm("" : "+v"(x));
+  return x;
 }
 
 template <typename TT>
@@ -137,7 +148,7 @@ __device__ void process_row(const AppendParams& p, const void* src, int64_t src_
   }
   auto fetch = [&](int e) -> float {
     float v = ldv<TT>(src, src_base + e);
-    if (norm_w) v = rnd<TT>(rnd<TT>(v * inv) * ldv<TT>(norm_w, e));
+    if (norm_w) v = rnd<TT>(rnd<TT>(mul32(v, inv)) * ldv<TT>(norm_w, e));
     return v;
   };
   auto put = [&](int e, float v) {
@@ -228,7 +239,7 @@ __device__ void int_row(const AppendParams& p, const void* src, int64_t sbase, v
   const int off = p.rotary_offset;
   auto fetch = [&](int e) -> float {
     float v = ldv<TT>(src, sbase + e);
-    if (norm_w) v = rnd<TT>(rnd<TT>(v * inv) * ldv<TT>(norm_w, e));
+    if (norm_w) v = rnd<TT>(rnd<TT>(mul32(v, inv)) * ldv<TT>(norm_w, e));
     return v;
   };
   auto value = [&](int e) -> float {
@@ -457,6 +468,342 @@ __global__ __launch_bounds__(256) void rotary_append_kernel(const AppendParams p
   }
 }
 
+// Two elements of T in one word.  pack2 rounds to nearest even, as TT::from_f32 does (bf16: one
+// v_cvt_pk_bf16_f32, equal to the integer rounding for every fp32 pattern, NaNs included).
+template <typename TT>
+struct Pair;
+template <>
+struct Pair<TF16> {
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  __device__ __forceinline__ static float lo(uint32_t w) { return TF16::to_f32((uint16_t)w); }
+  __device__ __forceinline__ static float hi(uint32_t w) { return TF16::to_f32((uint16_t)(w >> 16)); }
+  __device__ __forceinline__ static uint32_t pack2(float a, float b) {
+    return (uint32_t)TF16::from_f32(a) | ((uint32_t)TF16::from_f32(b) << 16);
+  }
+  // v c -+ w s, each operation rounded to fp16.  fp16 arithmetic gives the bits of an fp32
+  // operation rounded to fp16: products of two fp16 values are exact in fp32, and a sum or
+  // difference of two that falls near a rounding boundary of fp16 is exact there too.
+  __device__ __forceinline__ static uint32_t rope(uint32_t v, uint32_t w, uint32_t c, uint32_t s,
+                                                  bool first) {
+    const f16x2 x = __builtin_bit_cast(f16x2, v) * __builtin_bit_cast(f16x2, c);
+    const f16x2 y = __builtin_bit_cast(f16x2, w) * __builtin_bit_cast(f16x2, s);
+    return __builtin_bit_cast(uint32_t, first ? x - y : x + y);
+  }
+};
+template <>
+struct Pair<TBF16> {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  __device__ __forceinline__ static float lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
+  __device__ __forceinline__ static float hi(uint32_t w) {
+    return __builtin_bit_cast(float, w & 0xffff0000u);
+  }
+  __device__ __forceinline__ static uint32_t pack2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+  }
+  __device__ __forceinline__ static uint32_t rope(uint32_t v, uint32_t w, uint32_t c, uint32_t s,
+                                                  bool first) {
+    const uint32_t x = pack2(lo(v) * lo(c), hi(v) * hi(c));
+    const uint32_t y = pack2(lo(w) * lo(s), hi(w) * hi(s));
+    return first ? pack2(lo(x) - lo(y), hi(x) - hi(y)) : pack2(lo(x) + lo(y), hi(x) + hi(y));
+  }
+};
+// x * inv rounded to T, times the weight, rounded to T (process_row's norm).
+template <typename TT>
+__device__ __forceinline__ uint32_t norm2(uint32_t x, float inv, uint32_t w) {
+  using P = Pair<TT>;
+  const uint32_t y = P::pack2(mul32(P::lo(x), inv), mul32(P::hi(x), inv));
+  return P::pack2(P::lo(y) * P::lo(w), P::hi(y) * P::hi(w));
+}
+
+// Sum of squares of one row held as 8 elements per lane, RL lanes per row (RL = 8, 16 or 32, rows
+// aligned to RL lanes), in the order of sum_squares: virtual lane v = e % 64 folds its elements
+// e = v, v + 64, ... with fused multiply-adds -- lane group of 8 by lane group of 8, the running
+// fold passed 8 lanes on -- then the XOR butterfly over virtual distances 32, 16, 8 (real lanes 4,
+// 2, 1) and 4, 2, 1 (inside a lane).  Both partners of a butterfly pair add the same two values, so
+// the sum has the same bits as sum_squares'.
+template <int RL>
+__device__ __forceinline__ float row_sum_squares(const float (&x)[8], int lane) {
+  float a[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a[i] = __builtin_fmaf(x[i], x[i], 0.0f);
+#pragma unroll
+  for (int f = 1; f < RL / 8; ++f) {
+    const bool mine = ((lane & (RL - 1)) >> 3) == f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float before = __shfl(a[i], (lane - 8) & 63, 64);
+      if (mine) a[i] = __builtin_fmaf(x[i], x[i], before);
+    }
+  }
+#pragma unroll
+  for (int o = 4; o >= 1; o >>= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] += __shfl_xor(a[i], o, 64);
+#pragma unroll
+  for (int o = 4; o >= 1; o >>= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < o) a[i] += a[i + o];
+  return __shfl(a[0], lane | (RL - 1), 64);  // the last fold's lanes hold the whole row
+}
+
+// Append over 8-element chunks: Q/K RMSNorm + RoPE + cache store for 16-bit activations whose rows
+// split into 16-byte chunks (rows_append_takes names the conditions) and whose slots are distinct.
+// A token's chunks -- its query, key and value rows in turn -- go to the lanes of `slices`
+// wavefronts, each walking `passes` 64-lane passes of them: the sequence and slot lookups, the cos
+// and sin chunks and the norm weights (the same for every pass when a row is a power of two of
+// chunks) are fetched once per wavefront, and the next pass's rows are in flight while one is
+// rotated and stored.  A rotated chunk reads its partner chunk again (the same lines: L1 hits), so
+// no lane waits for another, and every access is 16 bytes (codes: 8 or 4).  The first rows load
+// before the lookups resolve.  The arithmetic is process_row's and int_row's, operation by
+// operation, so the bytes are the same.
+// RL: lanes per row (head_dim / 8) where it is a power of two (8, 16, 32: the norm's lane
+// exchanges need it), 0: any head_dim % 8 == 0, without norm.
+// HBM-bound on multi-token batches, latency-bound (cum -> block table -> store) on decode ones.
+// Against rotary_append_kernel (one wavefront per head row, 2 bytes per lane, a 64-bit division per
+// slot, integer bf16 rounding): 3079 tokens x 80 rows of head 64 (fp16, rotated; 63 MB moved) 73 ->
+// 16.9 us, 1098 x 48 rows of head 128 (bf16) 25.7 -> 12.1, decode steps of 64 tokens 6.9 -> 5.3 and
+// with int4 codes 8.8 -> 5.7, 64 latent tokens of 128 heads x 576 10.2 -> 9.2.  An unrolled form
+// with four passes in registers (159-190 VGPRs, 2-3 wavefronts per SIMD) took 33 us on the first;
+// the integer rounding alone cost 22 -> 12 us on the second.
+template <typename TT, int CK, int RL>
+__global__ __launch_bounds__(256) void rows_append_kernel(const AppendParams p, int slices,
+                                                          int passes) {
+  using raw = typename TT::raw;
+  const int lane = threadIdx.x & 63;
+  const int wid = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t = wid / slices, sl = wid - t * slices;
+  if (t >= p.num_tokens) return;  // whole wavefront
+  const bool linear = p.linear_cap > 0;
+  if (p.meta_out && wid == 0)
+    for (int i = lane; i <= p.batch; i += 64) {
+      p.meta_out[kMetaCum + i] = i * p.gqa_seq;  // cum
+      if (i < p.batch) {
+        const int li = p.seqlens_k[i] + 1;
+        if (p.ring_cap > 0) {
+          const RingGeom rg = ring_geom(li, p.gqa_seq, p.ring_cap, p.ring_window);
+          p.meta_out[meta_past(p.batch) + i] = rg.before;              // past (view rows)
+          p.meta_out[meta_keys(p.batch) + i] = rg.before + p.gqa_seq;  // key count
+          p.meta_out[meta_colofs(p.batch) + i] = rg.p - rg.before;     // bias column offset
+        } else {
+          p.meta_out[meta_past(p.batch) + i] = max(li - p.gqa_seq, 0);  // past (query_past)
+          p.meta_out[meta_keys(p.batch) + i] = li;                      // key count
+        }
+      }
+    }
+  const int D = RL ? 8 * RL : p.head_dim, cpr = RL ? RL : D / 8;
+  const bool do_q = p.do_q && (p.cos_cache != nullptr || p.q_norm != nullptr || p.copy_rows);
+  const int nqr = do_q ? p.num_heads : 0;  // query rows, then key rows, then value rows
+  const int nkr = (linear && p.gqa_kv_rows == 0) ? 0 : p.kv_heads;
+  const int nqk = nqr + nkr, nrows = nqk + (p.value ? nkr : 0);
+  const int off = p.rotary_offset, rhalf = p.cos_cache ? p.rotary_half : 0;
+
+  // Chunk of a pass: its row (nrows and beyond: none), first element, own and partner data.
+  struct Chunk {
+    int row, e;
+    u32x4 x, px;
+  };
+  auto partner = [&](int e) { return e - off < rhalf ? e + rhalf : e - rhalf; };
+  auto load = [&](int pass) __attribute__((always_inline)) {
+    Chunk c;
+    const int ch = (sl * passes + pass) * 64 + lane;
+    c.row = ch / cpr;
+    c.e = 8 * (ch - c.row * cpr);
+    c.x = c.px = u32x4{0u, 0u, 0u, 0u};
+    if (pass < passes && c.row < nrows) {
+      const raw* src =
+          c.row < nqr   ? reinterpret_cast<const raw*>(p.query) + (int64_t)t * p.q_ld + c.row * D
+          : c.row < nqk ? reinterpret_cast<const raw*>(p.key) + (int64_t)t * p.k_ld + (c.row - nqr) * D
+                        : reinterpret_cast<const raw*>(p.value) + (int64_t)t * p.v_ld + (c.row - nqk) * D;
+      c.x = *reinterpret_cast<const u32x4*>(src + c.e);
+      if (c.row < nqk && !p.rotary_interleaved && (unsigned)(c.e - off) < (unsigned)(2 * rhalf))
+        c.px = *reinterpret_cast<const u32x4*>(src + partner(c.e));
+    } else {
+      c.row = INT32_MAX;
+    }
+    return c;
+  };
+  Chunk cur = load(0), nxt = load(1);
+
+  // Positions and the cache slot (the rules of rotary_append_kernel).
+  int seq_b;
+  int64_t pos, rpos, slot;
+  if (linear) {
+    seq_b = t / p.gqa_seq;
+    const int j = t - seq_b * p.gqa_seq;
+    const int len = p.seqlens_k[seq_b] + 1;
+    const int qp = max(len - p.gqa_seq, 0);
+    pos = (int64_t)qp + j;
+    bool kv_store = p.gqa_kv_rows != 0 && j < len - qp;
+    rpos = pos;
+    if (p.ring_cap > 0) {
+      const RingGeom rg = ring_geom(len, p.gqa_seq, p.ring_cap, p.ring_window);
+      pos = (int64_t)rg.before + j;
+      rpos = (int64_t)rg.p + j;
+      kv_store = p.gqa_kv_rows != 0;
+    }
+    if (p.position_ids)
+      rpos = p.pos_offset_form ? p.position_ids[0] + j
+                               : p.position_ids[(int64_t)seq_b * p.gqa_seq + j];
+    slot = (kv_store && pos >= 0 && pos < p.linear_cap) ? pos : -1;
+  } else {
+    const SeqPos sp = seq_pos_of_token(p.cum, p.past, p.batch, t);
+    seq_b = sp.b;
+    pos = (int64_t)max(sp.past, 0) + (t - sp.start);
+    rpos = pos;
+    if (p.slot_mapping) {
+      slot = p.slot_mapping[t];
+    } else if ((p.block_size & (p.block_size - 1)) == 0) {  // slot_at without 64-bit divisions
+      const int sh = __builtin_ctz(p.block_size);
+      const int64_t bi = pos >> sh;
+      slot = -1;
+      if (bi < p.max_blocks) {
+        const int64_t blk = p.block_table[(int64_t)seq_b * p.max_blocks + bi];
+        if (blk >= 0 && blk < p.num_blocks) slot = (blk << sh) + (pos & (p.block_size - 1));
+      }
+    } else {
+      slot = slot_at(p, seq_b, pos);
+    }
+    if (slot >= p.num_blocks * p.block_size) slot = -1;
+  }
+  const bool store = slot >= 0;
+  const int half = (rpos >= 0 && rpos < p.rotary_positions) ? rhalf : 0;
+  const raw* cosr = reinterpret_cast<const raw*>(p.cos_cache) + (half ? rpos * half : 0);
+  const raw* sinr = reinterpret_cast<const raw*>(p.sin_cache) + (half ? rpos * half : 0);
+  constexpr int EB = CK == kCacheI4 ? 4 : CK == kCacheT ? 16 : 8;  // cache bytes per chunk
+  const int64_t blk = (CK == kCacheFp8 && store) ? (int64_t)((uint32_t)slot / (uint32_t)p.block_size) : 0;
+  auto elem = [](const u32x4& v, int k) -> float {
+    return TT::to_f32((raw)(v[k >> 1] >> (16 * (k & 1))));
+  };
+  // cos / sin of the chunk at element e (interleaved: four of each)
+  u32x4 cw = {0u, 0u, 0u, 0u}, sw = cw;
+  auto load_cs = [&](int e) __attribute__((always_inline)) {
+    const int rr = e - off;
+    if ((unsigned)rr >= (unsigned)(2 * half)) return;
+    if (p.rotary_interleaved) {
+      const u32x2 c = *reinterpret_cast<const u32x2*>(cosr + rr / 2);
+      const u32x2 s = *reinterpret_cast<const u32x2*>(sinr + rr / 2);
+      cw = u32x4{c[0], c[1], 0u, 0u};
+      sw = u32x4{s[0], s[1], 0u, 0u};
+    } else {
+      const int ri = rr < half ? rr : rr - half;
+      cw = *reinterpret_cast<const u32x4*>(cosr + ri);
+      sw = *reinterpret_cast<const u32x4*>(sinr + ri);
+    }
+  };
+  if constexpr (RL > 0) load_cs(8 * (lane & (RL - 1)));
+
+  for (int pass = 0; pass < passes; ++pass) {
+    const Chunk c = cur;
+    cur = nxt;
+    nxt = load(pass + 2);
+    const int r = c.row, e = c.e, rr = e - off;
+    const bool is_q = r < nqr, is_v = r >= nqk;
+    const bool rot = !is_v && (unsigned)rr < (unsigned)(2 * half);
+    if constexpr (RL == 0) load_cs(e);
+    float inv = 1.0f;
+    bool norm = false;
+    const raw* nw = nullptr;
+    if constexpr (RL > 0) {
+      if (p.q_norm) {  // every lane takes part in the exchanges
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = elem(c.x, k);
+        inv = 1.0f / __builtin_sqrtf(row_sum_squares<RL>(v, lane) / (float)D + p.norm_eps);
+        norm = !is_v;
+        nw = reinterpret_cast<const raw*>(is_q ? p.q_norm : p.k_norm);
+      }
+    }
+    if (r >= nrows) continue;
+    using P = Pair<TT>;
+    u32x4 y = c.x;
+    if (norm) {
+      const u32x4 w = *reinterpret_cast<const u32x4*>(nw + e);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) y[k] = norm2<TT>(y[k], inv, w[k]);
+    }
+    if (rot && p.rotary_interleaved) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float cc = elem(cw, k), s = elem(sw, k), a = P::lo(y[k]), b = P::hi(y[k]);
+        if (p.rope_fp32) {
+          y[k] = P::pack2(rot_sub32(a, cc, b, s), rot_add32(b, cc, a, s));
+        } else {
+          const uint32_t ac_bs = P::pack2(a * cc, b * s), bc_as = P::pack2(b * cc, a * s);
+          y[k] = P::pack2(P::lo(ac_bs) - P::hi(ac_bs), P::lo(bc_as) + P::hi(bc_as));
+        }
+      }
+    } else if (rot) {
+      const bool first = rr < half;
+      u32x4 w = c.px;
+      if (norm) {
+        const u32x4 pw = *reinterpret_cast<const u32x4*>(nw + partner(e));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = norm2<TT>(w[k], inv, pw[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (p.rope_fp32) {
+          const float a0 = P::lo(y[k]), b0 = P::lo(w[k]), c0 = P::lo(cw[k]), s0 = P::lo(sw[k]);
+          const float a1 = P::hi(y[k]), b1 = P::hi(w[k]), c1 = P::hi(cw[k]), s1 = P::hi(sw[k]);
+          y[k] = first ? P::pack2(rot_sub32(a0, c0, b0, s0), rot_sub32(a1, c1, b1, s1))
+                       : P::pack2(rot_add32(a0, c0, b0, s0), rot_add32(a1, c1, b1, s1));
+        } else {
+          y[k] = P::rope(y[k], w[k], cw[k], sw[k], first);
+        }
+      }
+    }
+    if (is_q) {
+      *reinterpret_cast<u32x4*>(reinterpret_cast<raw*>(p.q_out) +
+                                ((int64_t)t * p.num_heads + r) * D + e) = y;
+      continue;
+    }
+    const int kh = is_v ? r - nqk : r - nqr;
+    void* const rows_out = is_v ? p.v_out : p.k_out;
+    if (rows_out)
+      *reinterpret_cast<u32x4*>(reinterpret_cast<raw*>(rows_out) +
+                                ((int64_t)t * p.kv_heads + kh) * D + e) = y;
+    char* cache = reinterpret_cast<char*>(is_v ? p.value_cache : p.key_cache);
+    if (!store || !cache) continue;
+    const int64_t crow = linear ? ((int64_t)seq_b * p.kv_heads + kh) * p.linear_cap + slot
+                                : slot * p.kv_heads + kh;
+    char* dst = cache + (crow * cpr + e / 8) * EB;
+    if constexpr (CK == kCacheT) {
+      *reinterpret_cast<u32x4*>(dst) = y;
+    } else {
+      const float* sc = is_v ? p.v_scale : p.k_scale;
+      const bool pc = (is_v ? p.v_quant : p.k_quant) == PA_QUANT_PER_CHANNEL;
+      const bool recip = p.quant_reciprocal != 0;
+      uint32_t code[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const float f = elem(y, k);
+        if constexpr (CK == kCacheFp8) {
+          const float s8 = sc[blk * p.kv_heads + kh];
+          code[k] = s8 == 0.0f ? 0u : f32_to_e4m3_sat(f / s8);
+        } else {
+          const float si = sc[pc ? (int64_t)kh * D + e + k : 0];
+          code[k] = CK == kCacheI4
+                        ? (uint32_t)(int_code(f, si, recip, -8.0f, 7.0f) + 8)
+                        : (uint32_t)(uint8_t)(int8_t)int_code(f, si, recip, -128.0f, 127.0f);
+        }
+      }
+      if constexpr (CK == kCacheI4) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w |= (code[2 * k] | (code[2 * k + 1] << 4)) << (8 * k);
+        *reinterpret_cast<uint32_t*>(dst) = w;
+      } else {
+        u32x2 w = u32x2{0u, 0u};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w[k >> 2] |= (code[k] & 0xffu) << (8 * (k & 3));
+        *reinterpret_cast<u32x2*>(dst) = w;
+      }
+    }
+  }
+}
+
 // Plain append: no rotary or norm, cache in the activation dtype, paged, every token's slot
 // distinct (no last-writer rule) and every row 16-byte aligned.  One wavefront per token: the
 // key and value rows (all kv-heads, contiguous in the input and in the slot) are loaded 16
@@ -648,6 +995,92 @@ hipError_t launch_ring_move(const RingParams& r, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Whether [a, a + n) and [b, b + n) share no byte.
+static bool apart(const void* a, int64_t na, const void* b, int64_t nb) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return !a || !b || x + (uint64_t)na <= y || y + (uint64_t)nb <= x;
+}
+
+// Lanes per row of rows_append_kernel: head_dim / 8 where it is 8, 16 or 32, else 0.
+static int rows_append_lanes(int head_dim) {
+  return head_dim == 64 || head_dim == 128 || head_dim == 256 ? head_dim / 8 : 0;
+}
+
+// The calls that rows_append_kernel takes: 16-bit activations, distinct slots (paged caches with
+// the host's or the caller's word for it, contiguous ones by their layout), 16-byte chunks
+// everywhere (head_dim % 8, the rotary range and the row strides, every base address; code rows to
+// their 8 or 4 bytes), the norm only where a row fills 8, 16 or 32 lanes.  Rows whose chunks may
+// land in different wavefronts (RL = 0) re-read partner chunks after another wavefront may have
+// stored its own, so there the outputs must lie apart from the inputs.
+static bool rows_append_takes(const AppendParams& p, pa_dtype act, pa_dtype cache_dtype) {
+  if (act != PA_DTYPE_FLOAT16 && act != PA_DTYPE_BFLOAT16) return false;
+  const bool linear = p.linear_cap > 0;
+  if (!linear && !p.slots_distinct) return false;
+  if (!p.key && p.gqa_kv_rows) return false;
+  const int D = p.head_dim, rl = rows_append_lanes(D);
+  if (D % 8 != 0) return false;
+  const bool norm = p.q_norm != nullptr;
+  if (rl == 0 && (norm || cache_dtype != act)) return false;
+  if (p.cos_cache) {
+    if (p.rotary_offset % 8 != 0 || p.rotary_half % (p.rotary_interleaved ? 4 : 8) != 0)
+      return false;
+  }
+  const uintptr_t a16 = (uintptr_t)p.query | (uintptr_t)p.key | (uintptr_t)p.value |
+                        (uintptr_t)p.q_out | (uintptr_t)p.k_out | (uintptr_t)p.v_out |
+                        (uintptr_t)p.cos_cache | (uintptr_t)p.sin_cache | (uintptr_t)p.q_norm |
+                        (uintptr_t)p.k_norm | (uintptr_t)(p.q_ld * 2) | (uintptr_t)(p.k_ld * 2) |
+                        (uintptr_t)(p.v_ld * 2);
+  const uintptr_t ac = (uintptr_t)p.key_cache | (uintptr_t)p.value_cache;
+  const uintptr_t cb = cache_dtype == act ? 15 : cache_dtype == PA_DTYPE_INT4 ? 3 : 7;
+  if ((a16 & 15) != 0 || (ac & cb) != 0) return false;
+  if (cache_dtype != act && (!p.k_scale || !p.v_scale)) return false;
+  if (rl == 0) {
+    const int64_t nq = (int64_t)p.num_tokens * p.q_ld * 2, nk = (int64_t)p.num_tokens * p.k_ld * 2;
+    const int64_t oq = (int64_t)p.num_tokens * p.num_heads * D * 2;
+    const int64_t ok = (int64_t)p.num_tokens * p.kv_heads * D * 2;
+    if (!apart(p.query, nq, p.q_out, oq) || !apart(p.key, nk, p.k_out, ok)) return false;
+  }
+  return true;
+}
+
+constexpr int64_t kRowsWaves = 4096;
+template <typename TT, int CK, int RL>
+static void launch_rows(const AppendParams& p, hipStream_t s) {
+  const bool do_q = p.do_q && (p.cos_cache || p.q_norm || p.copy_rows);
+  const int kv = (p.linear_cap > 0 && p.gqa_kv_rows == 0) ? 0 : p.kv_heads;
+  const int64_t chunks =
+      ((int64_t)(do_q ? p.num_heads : 0) + kv + (p.value ? kv : 0)) * (p.head_dim / 8);
+  const int64_t per = std::max<int64_t>((chunks + 63) / 64, 1);  // 64-lane passes per token
+  // As many passes per wavefront as leave kRowsWaves wavefronts (8 per SIMD is what fits).
+  const int64_t want = (kRowsWaves + p.num_tokens - 1) / p.num_tokens;
+  const int passes = (int)std::max<int64_t>(per / std::max<int64_t>(want, 1), 1);
+  const int slices = (int)((per + passes - 1) / passes);
+  const dim3 grid((unsigned)(((int64_t)p.num_tokens * slices + 3) / 4));
+  hipLaunchKernelGGL((rows_append_kernel<TT, CK, RL>), grid, dim3(256), 0, s, p, slices, passes);
+}
+
+template <typename TT, int CK>
+static void launch_rows_ck(const AppendParams& p, hipStream_t s) {
+  switch (rows_append_lanes(p.head_dim)) {
+    case 8: launch_rows<TT, CK, 8>(p, s); break;
+    case 16: launch_rows<TT, CK, 16>(p, s); break;
+    case 32: launch_rows<TT, CK, 32>(p, s); break;
+    default:
+      if constexpr (CK == kCacheT) launch_rows<TT, CK, 0>(p, s);
+      break;
+  }
+}
+
+template <typename TT>
+static void launch_rows_t(const AppendParams& p, pa_dtype cache_dtype, hipStream_t s) {
+  switch (cache_dtype) {
+    case PA_DTYPE_FP8_E4M3: launch_rows_ck<TT, kCacheFp8>(p, s); break;
+    case PA_DTYPE_INT8: launch_rows_ck<TT, kCacheI8>(p, s); break;
+    case PA_DTYPE_INT4: launch_rows_ck<TT, kCacheI4>(p, s); break;
+    default: launch_rows_ck<TT, kCacheT>(p, s); break;
+  }
+}
+
 hipError_t launch_rotary_append(const AppendParams& p, pa_dtype act, pa_dtype cache_dtype,
                                 hipStream_t s) {
   if (p.num_tokens <= 0) return hipSuccess;
@@ -698,6 +1131,13 @@ hipError_t launch_rotary_append(const AppendParams& p, pa_dtype act, pa_dtype ca
       }
       return hipGetLastError();
     }
+  }
+  if (rows_append_takes(p, act, cache_dtype)) {
+    if (act == PA_DTYPE_FLOAT16)
+      launch_rows_t<TF16>(p, cache_dtype, s);
+    else
+      launch_rows_t<TBF16>(p, cache_dtype, s);
+    return hipGetLastError();
   }
   switch (act) {
     case PA_DTYPE_FLOAT16: launch_append_t<TF16>(p, cache_dtype, grid, block, s); break;
