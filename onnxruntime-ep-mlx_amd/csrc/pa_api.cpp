@@ -462,6 +462,70 @@ size_t workspace_for(const pa_cache* c, const pa_batch* b, const pa_attn*, const
   return n;
 }
 
+// A batch whose host metadata shows both decode sequences (at most 16 grouped query rows) and longer
+// ones, as a server with running and arriving requests sends: the decode sequences on the streaming
+// decode, the others on the prefill launches, over the same workspace in turn.  As one prefill batch
+// every decode sequence costs a 128-row item per kv-head and, with operand images, an image of its
+// whole context.
+struct SplitPlan {
+  bool on = false;
+  int short_tokens = 0;  // sequences of at most this many new tokens go to the decode
+  pa_batch dec_batch{}, pre_batch{};
+  Plan dec{}, pre{};
+  size_t seq_off = 0, bytes = 0;  // list of the prefill sequences, workspace in all
+};
+
+// Key/value bytes (as 16-bit rows) of the decode sequences from which a batch is split.  One launch
+// for all of them takes the planned prefill with fewer long rows than the long sequences alone need
+// for it, so small decode shares stay with it: with one prompt of 64 / 512 / 1500 tokens beside 48
+// contexts of 1000 (197 MB at 8 kv-heads of 128) 64.2 / 91.5 / 137.8 us split, 56.2 / 154.0 / 197.7
+// whole, 32 of 2000 (262 MB) 73.2 / 98.3 / 150.7 against 87.7 / 201.1 / 217.9; at head 256 48 of
+// 1000 beside 1500 tokens 238.7 against 215.4, 32 of 2000 230.7 against 257.9.  48 contexts of up
+// to 6000 and three prompts of up to 600 tokens: 390 -> 210 us a call.
+#ifndef PA_SPLIT_MIN_BYTES
+#define PA_SPLIT_MIN_BYTES (224ll << 20)
+#endif
+
+SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act,
+                     const HostLens& hl, bool images) {
+  SplitPlan sp;
+  if (!hl.cum || !hl.past || !c->value_cache || c->kv_heads < 1) return sp;
+  const int g = a->num_heads / c->kv_heads;
+  if (g < 1 || g > 16) return sp;
+  const int limit = 16 / g;
+  int n_long = 0, mq_short = 0, mq_long = 0;
+  int64_t keys = 0, ctx_long = 0;
+  for (int i = 0; i < b->batch; ++i) {
+    const int nq = hl.cum[i + 1] - hl.cum[i];
+    const int64_t ctx = (int64_t)std::max(hl.past[i], 0) + nq;
+    if (nq > limit) {
+      ++n_long;
+      mq_long = std::max(mq_long, nq);
+      ctx_long = std::max(ctx_long, ctx);
+    } else if (nq > 0) {
+      mq_short = std::max(mq_short, nq);
+      keys += a->local_window_size > 0 ? std::min<int64_t>(ctx, (int64_t)a->local_window_size + nq) : ctx;
+    }
+  }
+  if (n_long == 0 || n_long > pa::kMaxRanks || mq_short == 0 ||
+      keys * c->kv_heads * c->head_dim * 4 < (int64_t)PA_SPLIT_MIN_BYTES)
+    return sp;
+  sp.short_tokens = limit;
+  sp.dec_batch = sp.pre_batch = *b;
+  sp.dec_batch.max_query_len = mq_short;
+  sp.pre_batch.max_query_len = mq_long;
+  sp.pre_batch.max_context_len = (int32_t)std::min<int64_t>(ctx_long, INT32_MAX);
+  sp.pre_batch.batch = n_long;
+  sp.dec = make_plan(c, &sp.dec_batch, a, act, 0, 0, false, 0, images);
+  sp.pre = make_plan(c, &sp.pre_batch, a, act, 0, 0, false, 0, images);
+  if (!sp.dec.balanced || sp.pre.kind != 2 || sp.pre.sub_batch > 0) return sp;
+  sp.seq_off = workspace_for(c, &sp.pre_batch, a, sp.pre);
+  sp.bytes = std::max(workspace_for(c, &sp.dec_batch, a, sp.dec),
+                      sp.seq_off + align256((size_t)n_long * sizeof(int32_t)));
+  sp.on = true;
+  return sp;
+}
+
 // Options of one attention call beyond the public descriptors.
 struct RunOpts {
   bool new_rows_in_cache = false;  // new rows sit in their block-table slots (see AttnParams)
@@ -480,6 +544,97 @@ struct RunOpts {
 // take one -- the streaming decode and prefill_kernel -- read the cache rows themselves), so
 // byte-coded multi-token batches with a bias run on the VALU kernel.
 bool plan_images(const RunOpts& o) { return o.images && o.bias == nullptr; }
+
+// Kernel parameters of one launch (plan pl of batch b) of an attention call over workspace ws.
+pa::AttnParams attn_params(const pa_cache* c, const pa_batch* b, const pa_attn* a, const void* q,
+                           const void* kn, const void* vn, void* out, void* ws, const Plan& pl,
+                           const RunOpts& opts) {
+  const size_t need = workspace_for(c, b, a, pl);
+  const bool quant = c->dtype == PA_DTYPE_FP8_E4M3 || is_int_cache(c->dtype);
+  const bool latent = c->value_cache == nullptr;
+  pa::AttnParams p{};
+  p.q = q;
+  p.k_new = kn;
+  p.v_new = vn;
+  p.key_cache = c->key_cache;
+  p.value_cache = c->value_cache;
+  p.k_scale = c->k_scale;
+  p.v_scale = c->v_scale;
+  p.cum = b->cumulative_sequence_length;
+  p.past = b->past_seqlens;
+  p.block_table = b->block_table;
+  p.head_sink = a->head_sink;
+  p.out = out;
+  p.part_o = need ? reinterpret_cast<float*>(ws) : nullptr;
+  p.part_ml = need ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + part_o_bytes(c, pl))
+                   : nullptr;
+  if (pl.plan_items > 0) {
+    char* base = reinterpret_cast<char*>(ws) + part_o_bytes(c, pl) +
+                 align256(pl.part_rows * 2 * sizeof(float));
+    p.plan = reinterpret_cast<int32_t*>(base);
+    base += align256((size_t)pl.plan_items * 2 * 4 * sizeof(int32_t));
+    p.plan_info = reinterpret_cast<int32_t*>(base);
+    p.plan_split = reinterpret_cast<int32_t*>(base + 256);
+    p.plan_items = (int32_t)pl.plan_items;
+    p.plan_rbs = pl.plan_rbs;
+    // workgroups resident per CU: two, three for the 32-key image kernel (148 VGPRs, 33 KB LDS),
+    // one for the bias kernel from head 128 on
+    p.plan_slots = (pl.img_steps > 0 && pa::img_keys(c->head_dim) == 32 && c->head_dim <= 128
+                        ? PA_IMG_WAVES
+                    : opts.bias && c->head_dim >= 128 ? 1
+                                                      : 2) * device_cus();
+    p.plan_step = pl.img_steps > 0 ? pa::img_keys(c->head_dim) : pa::prefill_key_step(c->head_dim);
+    if (pl.img_steps > 0) {
+      const size_t hb = (size_t)plan_batch(b, pl) * c->kv_heads;
+      char* img = base + plan_bytes(pl) - align256((size_t)pl.plan_items * 2 * 4 * sizeof(int32_t));
+      p.vimg = img;
+      img += align256(hb * pl.img_steps * pa::img_step_bytes(c->head_dim));
+      p.vstep = reinterpret_cast<int32_t*>(img);
+      img += align256(hb * pl.img_steps * sizeof(int32_t));
+      p.img_wide = reinterpret_cast<int32_t*>(img);
+      p.img_epoch = next_img_epoch();
+      p.img_steps = pl.img_steps;
+    }
+  }
+  p.num_blocks = c->num_blocks;
+  p.block_size = c->block_size;
+  p.kv_heads = c->kv_heads;
+  p.head_dim = c->head_dim;
+  p.num_heads = a->num_heads;
+  p.batch = p.seqs = b->batch;
+  p.max_blocks = b->max_blocks;
+  p.num_tokens = b->num_tokens;
+  p.chunk = pl.chunk;
+  p.max_splits = pl.max_splits;
+  p.mix = pl.mix;
+  p.linear_cap = opts.linear_cap;
+  p.ng = pl.ng > 0 ? pl.ng : 1;
+  p.max_query_len = b->max_query_len > 0 ? b->max_query_len : b->num_tokens;
+  p.scale = a->scale != 0.0f ? a->scale : 1.0f / std::sqrt((float)c->head_dim);
+  p.scale_log2 = p.scale * pa::kLog2e;
+  p.softcap = a->softcap;
+  p.window = a->local_window_size;
+  p.causal = a->is_causal ? 1 : 0;
+  p.read_all_from_cache = quant ? 1 : 0;
+  p.k_quant = c->k_quant_type;
+  p.v_quant = c->v_quant_type;
+  p.v_head_dim = a->v_head_size > 0 ? a->v_head_size : c->head_dim;
+  p.v_from_key = latent ? 1 : 0;
+  p.new_rows_in_cache =
+      (opts.new_rows_in_cache || ((b->flags & PA_BATCH_NEW_ROWS_IN_CACHE) && !b->slot_mapping))
+          ? 1
+          : 0;
+  p.key_limit = opts.key_limit;
+  p.bias = opts.bias;
+  p.bias_b = opts.bias_b;
+  p.bias_h = opts.bias_h;
+  p.bias_rows = opts.bias_rows;
+  p.bias_cols = opts.bias_cols;
+  p.bias_col_off = opts.bias_col_off;
+  p.smooth_softmax = opts.smooth_softmax ? 1 : 0;
+
+  return p;
+}
 
 int run_attention(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act,
                   const void* q, const void* kn, const void* vn, void* out, void* ws,
@@ -534,87 +689,24 @@ int run_attention(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dty
     return fail(PA_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes, got %zu", need,
                 ws_bytes);
 
-  pa::AttnParams p{};
-  p.q = q;
-  p.k_new = kn;
-  p.v_new = vn;
-  p.key_cache = c->key_cache;
-  p.value_cache = c->value_cache;
-  p.k_scale = c->k_scale;
-  p.v_scale = c->v_scale;
-  p.cum = b->cumulative_sequence_length;
-  p.past = b->past_seqlens;
-  p.block_table = b->block_table;
-  p.head_sink = a->head_sink;
-  p.out = out;
-  p.part_o = need ? reinterpret_cast<float*>(ws) : nullptr;
-  p.part_ml = need ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + part_o_bytes(c, pl))
-                   : nullptr;
-  if (pl.plan_items > 0) {
-    char* base = reinterpret_cast<char*>(ws) + part_o_bytes(c, pl) +
-                 align256(pl.part_rows * 2 * sizeof(float));
-    p.plan = reinterpret_cast<int32_t*>(base);
-    base += align256((size_t)pl.plan_items * 2 * 4 * sizeof(int32_t));
-    p.plan_info = reinterpret_cast<int32_t*>(base);
-    p.plan_split = reinterpret_cast<int32_t*>(base + 256);
-    p.plan_items = (int32_t)pl.plan_items;
-    p.plan_rbs = pl.plan_rbs;
-    // workgroups resident per CU: two, three for the 32-key image kernel (148 VGPRs, 33 KB LDS),
-    // one for the bias kernel from head 128 on
-    p.plan_slots = (pl.img_steps > 0 && pa::img_keys(c->head_dim) == 32 && c->head_dim <= 128
-                        ? PA_IMG_WAVES
-                    : opts.bias && c->head_dim >= 128 ? 1
-                                                      : 2) * device_cus();
-    p.plan_step = pl.img_steps > 0 ? pa::img_keys(c->head_dim) : pa::prefill_key_step(c->head_dim);
-    if (pl.img_steps > 0) {
-      const size_t hb = (size_t)plan_batch(b, pl) * c->kv_heads;
-      char* img = base + plan_bytes(pl) - align256((size_t)pl.plan_items * 2 * 4 * sizeof(int32_t));
-      p.vimg = img;
-      img += align256(hb * pl.img_steps * pa::img_step_bytes(c->head_dim));
-      p.vstep = reinterpret_cast<int32_t*>(img);
-      img += align256(hb * pl.img_steps * sizeof(int32_t));
-      p.img_wide = reinterpret_cast<int32_t*>(img);
-      p.img_epoch = next_img_epoch();
-      p.img_steps = pl.img_steps;
-    }
+  const bool whole = kind == 0 && chunk == 0 && opts.linear_cap == 0;
+  const SplitPlan sp = whole ? split_plan(c, b, a, act, opts.host, plan_images(opts)) : SplitPlan();
+  if (sp.on && ws_bytes >= sp.bytes) {
+    pa::AttnParams pd = attn_params(c, &sp.dec_batch, a, q, kn, vn, out, ws, sp.dec, opts);
+    pa::AttnParams pp = attn_params(c, &sp.pre_batch, a, q, kn, vn, out, ws, sp.pre, opts);
+    pd.short_tokens = pp.short_tokens = sp.short_tokens;
+    pp.batch = b->batch;  // (seqs: the prefill's share)
+    pp.plan_seq = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(ws) + sp.seq_off);
+    hipError_t e = pa::launch_decode_balanced(pd, act, c->dtype, s);
+    if (e != hipSuccess) return hip_fail(e, "balanced decode launch");
+    e = sp.pre.plan_items > 0 ? pa::launch_prefill_planned(pp, act, c->dtype, s)
+                              : pa::launch_prefill_mfma(pp, act, c->dtype, s);
+    if (e == hipSuccess && sp.pre.max_splits > 1) e = pa::launch_split_reduce(pp, act, s);
+    if (e != hipSuccess) return hip_fail(e, "attention kernel launch");
+    return PA_OK;
   }
-  p.num_blocks = c->num_blocks;
-  p.block_size = c->block_size;
-  p.kv_heads = c->kv_heads;
-  p.head_dim = c->head_dim;
-  p.num_heads = a->num_heads;
-  p.batch = b->batch;
-  p.max_blocks = b->max_blocks;
-  p.num_tokens = b->num_tokens;
-  p.chunk = pl.chunk;
-  p.max_splits = pl.max_splits;
-  p.mix = pl.mix;
-  p.linear_cap = opts.linear_cap;
-  p.ng = pl.ng > 0 ? pl.ng : 1;
-  p.max_query_len = b->max_query_len > 0 ? b->max_query_len : b->num_tokens;
-  p.scale = a->scale != 0.0f ? a->scale : 1.0f / std::sqrt((float)c->head_dim);
-  p.scale_log2 = p.scale * pa::kLog2e;
-  p.softcap = a->softcap;
-  p.window = a->local_window_size;
-  p.causal = a->is_causal ? 1 : 0;
-  p.read_all_from_cache = quant ? 1 : 0;
-  p.k_quant = c->k_quant_type;
-  p.v_quant = c->v_quant_type;
-  p.v_head_dim = vd;
-  p.v_from_key = latent ? 1 : 0;
-  p.new_rows_in_cache =
-      (opts.new_rows_in_cache || ((b->flags & PA_BATCH_NEW_ROWS_IN_CACHE) && !b->slot_mapping))
-          ? 1
-          : 0;
-  p.key_limit = opts.key_limit;
-  p.bias = opts.bias;
-  p.bias_b = opts.bias_b;
-  p.bias_h = opts.bias_h;
-  p.bias_rows = opts.bias_rows;
-  p.bias_cols = opts.bias_cols;
-  p.bias_col_off = opts.bias_col_off;
-  p.smooth_softmax = opts.smooth_softmax ? 1 : 0;
 
+  const pa::AttnParams p = attn_params(c, b, a, q, kn, vn, out, ws, pl, opts);
   hipError_t e;
   if (pl.balanced) {
     e = pa::launch_decode_balanced(p, act, c->dtype, s);  // attention + partial merge
@@ -634,7 +726,7 @@ int run_attention(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dty
           q.cum = p.cum + b0;
           q.past = p.past + b0;
           q.block_table = p.block_table + b0 * p.max_blocks;
-          q.batch = nb;
+          q.batch = q.seqs = nb;
           q.plan_items = (int32_t)((int64_t)nb * c->kv_heads * pl.plan_rbs);
           if (p.key_limit) q.key_limit = p.key_limit + b0;
           // fresh wide-step flags: the image slots are reused by every group
@@ -883,6 +975,7 @@ struct OpLayout {
   int head, v_head, kv_hidden;
   bool packed, transform;
   size_t q_bytes, k_bytes, v_bytes, attn_off, total;
+  size_t best;  // with this much the call may split its batch (split_plan); total is enough to run
   pa_batch batch;
   pa_attn attn;
 };
@@ -982,6 +1075,11 @@ int op_layout(const pa_paged_attention_node* n, const pa_paged_attention_io* io,
                                      false,
                                      HostLens{io->host_cumulative_sequence_length,
                                               io->host_past_seqlens}));
+  const SplitPlan sp = split_plan(&io->cache, &b, &a, io->dtype,
+                                  HostLens{io->host_cumulative_sequence_length,
+                                           io->host_past_seqlens},
+                                  images);
+  L->best = std::max(L->total, sp.on ? L->attn_off + sp.bytes : 0);
   return PA_OK;
 }
 
@@ -1118,7 +1216,7 @@ size_t pa_paged_attention_workspace_bytes(const pa_paged_attention_node* node,
                                           const pa_paged_attention_io* io) {
   OpLayout L;
   if (op_layout(node, io, &L)) return 0;
-  return L.total;
+  return L.best;
 }
 
 // The operator entry; images: see make_plan.

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(NT) void split_reduce_kernel(const AttnParams p) {
   const int b = seq_of_token(p.cum, p.batch, t);
   const int nq = p.cum[b + 1] - p.cum[b];
   const int64_t total = seq_keys(p, b, max(p.past[b], 0), nq);
-  if (nq <= 0) return;
+  if (nq <= 0 || nq <= p.short_tokens) return;  // (short: a row of the streaming decode)
   const int nsplit = (int)min((total + p.chunk - 1) / p.chunk, (int64_t)p.max_splits);
   if (nsplit <= 1) return;  // the attention kernel already wrote the final row
   const int64_t base = ((int64_t)t * p.num_heads + h) * p.max_splits;

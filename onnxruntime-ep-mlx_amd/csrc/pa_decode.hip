@@ -457,6 +457,7 @@ __device__ __forceinline__ SeqSteps seq_steps(const AttnParams& p, int b) {
                                    : (int)min((int64_t)p.max_blocks * p.block_size,
                                               (int64_t)(INT32_MAX / 2));
   q.nq = min(s1 - q.s0, cap);
+  if (p.short_tokens > 0 && q.nq > p.short_tokens) q.nq = 0;  // a sequence of the prefill launches
   const bool any = q.nq > 0;
   q.pastb = any ? min(max(pb, 0), cap - q.nq) : 0;
   q.total = any ? q.pastb + q.nq : 0;

@@ -385,7 +385,18 @@ struct AttnParams {
   // of the pair is wide (bf16 values kept raw, see the image writer); any other value: none
   int32_t* img_wide;
   int32_t img_epoch;
+  // A batch split by query length (short_tokens > 0): the sequences of at most short_tokens new
+  // tokens belong to the streaming decode, which takes no steps of the others, and the others --
+  // `seqs` of them, in batch order -- to the prefill launches, whose sequence index n is then a
+  // rank among them (seq_of_rank; plan_seq[n] once the plan kernel has run, -1 past the last one).
+  // short_tokens == 0: every launch takes every sequence, n is the sequence and seqs == batch.
+  int32_t short_tokens, seqs;
+  int32_t* plan_seq;
 };
+
+// Sequences of the prefill launches of a batch split by query length, at most (the plan kernel
+// holds their list in LDS).
+constexpr int kMaxRanks = 1024;
 
 // Image geometry of the planned prefill: kImgKeys keys x d dims of 16-bit keys and values per
 // step (the prefill kernel's key step over images: 32 or 64).

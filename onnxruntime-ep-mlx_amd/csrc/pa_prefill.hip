@@ -215,13 +215,15 @@ prefill_kernel(const AttnParams p) {
     kh = item % p.kv_heads;
     rb = (item / p.kv_heads) % p.plan_rbs;
     b = item / (p.kv_heads * p.plan_rbs);
+    if (p.short_tokens > 0) b = p.plan_seq[b];
   } else {
-    const int units = p.batch * p.kv_heads;
+    const int units = p.seqs * p.kv_heads;
     const int unit = blockIdx.x % units;
     rb = (int)(gridDim.x / units) - 1 - (int)(blockIdx.x / units);
     kh = unit % p.kv_heads;
-    b = unit / p.kv_heads;
+    b = seq_of_rank(p, unit / p.kv_heads);
   }
+  if (b < 0) return;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, G = lane >> 4;
   // Everything up to the first barrier is uniform over the workgroup.
   const int s0 = min(max(p.cum[b], 0), p.num_tokens);
@@ -643,7 +645,7 @@ prefill_mx_kernel(const AttnParams p) {
   constexpr int KB = IMG ? img_keys(D) / 32 : 2, KEYS = 32 * KB, KS = D / 16, NQ = D / 32;
   using Buf = MxBufT<KB, D>;
   __shared__ Buf lds[2];
-  int rb, kh, b, split = blockIdx.y, part = 0, item = 0, ustart = 0, uend = 0;
+  int rb, kh, b, rank, split = blockIdx.y, part = 0, item = 0, ustart = 0, uend = 0;
   if (p.plan_items > 0) {
     const int nunits = p.plan_info[0];
     const int4 u = reinterpret_cast<const int4*>(p.plan)[min((int)blockIdx.x, p.plan_items * 2 - 1)];
@@ -654,14 +656,17 @@ prefill_mx_kernel(const AttnParams p) {
     uend = u.w;
     kh = item % p.kv_heads;
     rb = (item / p.kv_heads) % p.plan_rbs;
-    b = item / (p.kv_heads * p.plan_rbs);
+    rank = item / (p.kv_heads * p.plan_rbs);
+    b = p.short_tokens > 0 ? p.plan_seq[rank] : rank;
   } else {
-    const int units = p.batch * p.kv_heads;
+    const int units = p.seqs * p.kv_heads;
     const int unit = blockIdx.x % units;
     rb = (int)(gridDim.x / units) - 1 - (int)(blockIdx.x / units);
     kh = unit % p.kv_heads;
-    b = unit / p.kv_heads;
+    rank = unit / p.kv_heads;
+    b = seq_of_rank(p, rank);
   }
+  if (b < 0) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   const int s0 = min(max(p.cum[b], 0), p.num_tokens);
@@ -983,7 +988,7 @@ prefill_mx_kernel(const AttnParams p) {
   auto seen = [&](int t0) { return t0 < any_hi && t0 + KEYS > any_lo; };
 
   if constexpr (IMG) {
-    const int64_t hb = (int64_t)b * p.kv_heads + kh;
+    const int64_t hb = (int64_t)rank * p.kv_heads + kh;
     const char* img_hb = p.vimg + hb * p.img_steps * (int64_t)img_step_bytes(D);
     const int32_t* vstep_hb = p.vstep + hb * p.img_steps;
     // Direct LDS loads of step k + 1 into the other buffer while step k computes (every
@@ -1154,9 +1159,12 @@ prefill_mx_kernel(const AttnParams p) {
 struct ItemKeys {
   int first, end;
 };
-__device__ __forceinline__ ItemKeys item_keys(const AttnParams& p, int i) {
+// `seqs` (a batch split by query length): the sequence of each rank.
+__device__ __forceinline__ ItemKeys item_keys(const AttnParams& p, int i, const int* seqs) {
   const int g = p.num_heads / p.kv_heads;
-  const int rb = (i / p.kv_heads) % p.plan_rbs, b = i / (p.kv_heads * p.plan_rbs);
+  const int rb = (i / p.kv_heads) % p.plan_rbs, n = i / (p.kv_heads * p.plan_rbs);
+  const int b = p.short_tokens > 0 ? seqs[n] : n;
+  if (b < 0) return ItemKeys{0, -1};
   const int s0 = min(max(p.cum[b], 0), p.num_tokens);
   const int s1 = min(max(p.cum[b + 1], s0), p.num_tokens);
   const int R = g * (s1 - s0);
@@ -1260,15 +1268,16 @@ __device__ __forceinline__ void img_load(const AttnParams& p, int id, ImgGroup<N
   constexpr int SPW = NT / 256, KEYS = img_keys(D), PCS = ImgGroup<NT, D>::PCS;
   constexpr int CH = ImgGroup<NT, D>::CH;
   const int nj = (p.img_steps + SPW - 1) / SPW;
-  const int jb = id % nj, kh = (id / nj) % p.kv_heads, b = min(id / (nj * p.kv_heads), p.batch - 1);
+  const int jb = id % nj, kh = (id / nj) % p.kv_heads, rank = min(id / (nj * p.kv_heads), p.seqs - 1);
+  const int bn = seq_of_rank(p, __builtin_amdgcn_readfirstlane(rank)), b = max(bn, 0);
   const int s0 = min(max(p.cum[b], 0), p.num_tokens);
-  const int s1 = min(max(p.cum[b + 1], s0), p.num_tokens);
+  const int s1 = bn < 0 ? s0 : min(max(p.cum[b + 1], s0), p.num_tokens);
   const int pastb = clamped_past(p, b, s1 - s0);
   const int total = seq_total(p, b, pastb, s1 - s0);
   const int tid = threadIdx.x;
   g.j = jb * SPW + tid / 256;
   g.step_live = s1 > s0 && g.j < p.img_steps && g.j * KEYS < total;
-  g.hb = (int64_t)b * p.kv_heads + kh;
+  g.hb = (int64_t)rank * p.kv_heads + kh;
   g.r = (tid & 255) / PCS;
   g.q = tid % PCS;
   WaveInfo w = make_wave(p, D, b, kh, s0, pastb, total);
@@ -1476,7 +1485,7 @@ __device__ __forceinline__ void image_steps(const AttnParams& p, int id) {
   __shared__ uint32_t rows[SPW][img_keys(D)][D / 2 + 1];  // fp16 value rows, one word = two dims
   __shared__ int emax[2 * SPW];  // per step: value exponent, then (fp8 pages) key exponent
   const int nj = (p.img_steps + SPW - 1) / SPW;
-  if (id >= nj * p.kv_heads * p.batch) return;
+  if (id >= nj * p.kv_heads * p.seqs) return;
   ImgGroup<NT, D> g;
   img_load<NT, D, KC>(p, id, g);
   img_store<TT, NT, D, KC>(p, g, rows, emax);
@@ -1496,15 +1505,30 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
   const int tid = threadIdx.x;
   for (int i = tid; i < NB; i += NT) hist[i] = 0;
   if (tid == 0) total_keys = 0;
+  // A batch split by query length: the sequences of the prefill ranks, for this kernel and, as
+  // plan_seq, for the launches behind it (one wavefront, in batch order).
+  __shared__ int seqs[kMaxRanks];
+  if (p.short_tokens > 0 && tid < 64) {
+    int n = 0;
+    for (int base = 0; base < p.batch; base += 64) {
+      const int b = base + tid;
+      const bool is = b < p.batch && seq_tokens(p, min(b, p.batch - 1)) > p.short_tokens;
+      const uint64_t m = __ballot(is);
+      const int at = n + __builtin_popcountll(m & ((1ull << tid) - 1));
+      if (is && at < p.seqs) seqs[at] = p.plan_seq[at] = b;
+      n += __builtin_popcountll(m);
+    }
+    for (int at = n + tid; at < p.seqs; at += 64) seqs[at] = p.plan_seq[at] = -1;
+  }
   __syncthreads();
   // The key ranges of this thread's first kCached items stay in registers for the later passes
   // (each costs two dependent metadata loads).
   constexpr int kCached = 4;
   ItemKeys cached[kCached];
-  auto keys = [&](int j, int i) { return j < kCached ? cached[j] : item_keys(p, i); };
+  auto keys = [&](int j, int i) { return j < kCached ? cached[j] : item_keys(p, i, seqs); };
   unsigned long long mine = 0;
   for (int i = tid, j = 0; i < p.plan_items; i += NT, ++j) {
-    const ItemKeys k = item_keys(p, i);
+    const ItemKeys k = item_keys(p, i, seqs);
 #pragma unroll
     for (int c = 0; c < kCached; ++c)
       if (c == j) cached[c] = k;
@@ -1608,7 +1632,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p) 
   if (!p.plan_split[i]) return;
   const int g = p.num_heads / p.kv_heads;
   const int kh = i % p.kv_heads, rb = (i / p.kv_heads) % p.plan_rbs;
-  const int b = i / (p.kv_heads * p.plan_rbs);
+  int b = i / (p.kv_heads * p.plan_rbs);
+  if (p.short_tokens > 0) b = p.plan_seq[b];  // (a split item's rank always has a sequence)
   const int row0 = rb * kPrefillRows;
   const int q = threadIdx.x % QPR;
   const int rbase = (blockIdx.x % CH) * kPrefillMergeRows + threadIdx.x / QPR;
@@ -1756,12 +1781,14 @@ hipError_t launch_prefill_planned(const AttnParams& p, pa_dtype act, pa_dtype ca
       !p.plan_split || !p.part_o || !p.part_ml || p.max_splits != 1)
     return hipErrorInvalidValue;
   if ((int64_t)p.plan_items * (kPrefillRows / kPrefillMergeRows) > INT32_MAX) return hipErrorInvalidValue;
+  if (p.seqs < 1 || (p.short_tokens > 0 && (!p.plan_seq || p.seqs > kMaxRanks)))
+    return hipErrorInvalidValue;
   // Operand images: written by workgroups 1.. of the plan launch.
   constexpr int kPlanThreads = 1024;
   const bool img = p.vimg != nullptr;
   if (img && (!img_head(p.head_dim) || !p.vstep || p.img_steps <= 0))
     return hipErrorInvalidValue;
-  const int64_t nimg = img ? (int64_t)p.batch * p.kv_heads *
+  const int64_t nimg = img ? (int64_t)p.seqs * p.kv_heads *
                                  ((p.img_steps + kPlanThreads / 256 - 1) / (kPlanThreads / 256))
                            : 0;
   if (nimg + 1 > INT32_MAX) return hipErrorInvalidValue;
@@ -1838,7 +1865,8 @@ hipError_t launch_prefill_mfma(const AttnParams& p, pa_dtype act, pa_dtype cache
   const int g = p.num_heads / p.kv_heads;
   const int mq = p.max_query_len > 0 ? p.max_query_len : p.num_tokens;
   const int64_t rbs = ((int64_t)g * mq + kPrefillRows - 1) / kPrefillRows;
-  const int64_t units = (int64_t)p.batch * p.kv_heads;
+  const int64_t units = (int64_t)p.seqs * p.kv_heads;
+  if (p.seqs < 1) return hipErrorInvalidValue;
   if (rbs * units > INT32_MAX || p.max_splits > 65535) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(rbs * units), p.max_splits);
   if (act == PA_DTYPE_FLOAT16) return launch_t<TF16>(p, grid, s);

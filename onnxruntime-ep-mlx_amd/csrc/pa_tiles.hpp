@@ -461,6 +461,30 @@ __device__ __forceinline__ int clamped_past(const AttnParams& p, int b, int nq) 
   return min(max(p.past[b], 0), max(cap - nq, 0));
 }
 
+// Query tokens of sequence b, as the device metadata has them.
+__device__ __forceinline__ int seq_tokens(const AttnParams& p, int b) {
+  const int s0 = min(max(p.cum[b], 0), p.num_tokens);
+  return min(max(p.cum[b + 1], s0), p.num_tokens) - s0;
+}
+
+// Sequence of prefill rank n (AttnParams::short_tokens), -1 if the batch holds fewer.  Run by whole
+// wavefronts with a uniform n: 64 sequences are tested at a time.
+__device__ __forceinline__ int seq_of_rank(const AttnParams& p, int n) {
+  if (p.short_tokens == 0) return n;
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < p.batch; base += 64) {
+    const int b = base + lane;
+    uint64_t m = __ballot(b < p.batch && seq_tokens(p, min(b, p.batch - 1)) > p.short_tokens);
+    const int c = __builtin_popcountll(m);
+    if (n < c) {
+      for (; n > 0; --n) m &= m - 1;
+      return base + __builtin_ctzll(m);
+    }
+    n -= c;
+  }
+  return -1;
+}
+
 // Keys of sequence b: past + query rows, bounded by key_limit[b] when given (GroupQueryAttention
 // first prompts whose sequences are shorter than the padded query rows).
 __device__ __forceinline__ int seq_total(const AttnParams& p, int b, int pastb, int nq) {
