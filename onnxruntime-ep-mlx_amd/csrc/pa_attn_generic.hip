@@ -1,7 +1,8 @@
 // pa_attn_generic.hip — VALU paged attention for every dtype/shape, plus the split-K reduce.
 //
-// One wavefront per (packed query token, query head, context chunk).  Lanes split head_dim;
-// each key costs one cross-lane sum.  This is the fp32 path (the ORT CPU GQA parity config)
+// One workgroup of NW wavefronts per (packed query token, query head, context chunk).  Lanes split
+// head_dim; each key costs one cross-lane sum.  The wavefronts take keys in turn, several of them
+// in flight, and meet in LDS at the end.  This is the fp32 path (the ORT CPU GQA parity config)
 // and the fallback for shapes the MFMA kernels do not cover, including integer (int8/int4)
 // pages, whose keys/values are code * scale in fp32; it is not the hot path.
 //
@@ -83,10 +84,19 @@ template <>
 constexpr bool kIntCache<I4Cache> = true;
 
 // Elements per lane: NE = 4 covers head_dim <= 256, NE = 10 head_dim <= 640 (latent heads).
-template <typename TT, typename CT, int NE>
-__global__ __launch_bounds__(64) void attn_generic_kernel(const AttnParams p) {
+// NW wavefronts take keys w, w + NW, ... of the chunk, kGenKeys of them per round: their rows are
+// loaded together and their cross-lane sums interleave.  A round is a chain of two or three memory
+// latencies (block table, rows) and the sums, so a call of few (token, head) pairs takes as long as
+// its rounds: one fp32 token of 8 heads over 129 keys 79 us with one wavefront and one key at a
+// time, 10.8 with 16 (launch_generic_ne has the rule).
+template <int NE>
+constexpr int kGenKeys = NE <= 4 ? 8 : 2;
+template <typename TT, typename CT, int NE, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_generic_kernel(const AttnParams p) {
+  constexpr int U = kGenKeys<NE>;
   const int split = blockIdx.x, h = blockIdx.y, t = blockIdx.z;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int D = p.head_dim;
   const int VD = p.v_head_dim;  // value / output head size (< D only for the LATENT layout)
   const int b = seq_of_token(p.cum, p.batch, t);
@@ -133,61 +143,116 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(const AttnParams p) {
   }
   float m = kNegInf, l = 0.0f;
   const float cap = p.softcap;
-  for (int64_t pos = lo; pos < hi; ++pos) {
-    const void *kb, *vb;
-    int64_t off;
-    float ks = 1.0f, vs = 1.0f;
-    bool from_cache = pos < pastb || p.read_all_from_cache || p.linear_cap > 0;
-    if (p.linear_cap > 0) {
-      // contiguous [batch, kv_heads, cap, head_dim] cache holding the new rows too
-      off = (((int64_t)b * p.kv_heads + kh) * p.linear_cap + pos) * Dc;
-      kb = p.key_cache;
-      vb = p.v_from_key ? p.key_cache : p.value_cache;
-    } else if (from_cache) {
-      int64_t bi = pos / p.block_size;
-      int64_t blk = p.block_table[(int64_t)b * p.max_blocks + min(bi, (int64_t)p.max_blocks - 1)];
-      blk = min(max(blk, (int64_t)0), p.num_blocks - 1);
-      off = (blk * p.block_size + pos % p.block_size) * crow + (int64_t)kh * Dc;
-      kb = p.key_cache;
-      vb = p.v_from_key ? p.key_cache : p.value_cache;
-      if (std::is_same<CT, Fp8Cache>::value) {
-        ks = p.k_scale[blk * p.kv_heads + kh];
-        vs = p.v_scale[blk * p.kv_heads + kh];
-      }
-    } else {
-      int64_t tok = min(max((int64_t)s0 + (pos - pastb), (int64_t)0), (int64_t)p.num_tokens - 1);
-      off = tok * row + (int64_t)kh * D;
-      kb = p.k_new;
-      vb = p.v_from_key ? p.k_new : p.v_new;
-    }
-    float part = 0.0f;
+  for (int64_t p0 = lo + wave; p0 < hi; p0 += NW * U) {
+    float x[U], vv[U][NE];
+    {
+      float part[U];
 #pragma unroll
-    for (int k = 0; k < NE; ++k) {
-      int e = lane + 64 * k;
-      if (e < D) {
-        float kv = from_cache ? CacheRead<CT>::at(kb, off, e, kIntCache<CT> ? ksv[k] : ks)
-                              : TT::to_f32(reinterpret_cast<const typename TT::raw*>(kb)[off + e]);
-        part += qv[k] * kv;
+      for (int u = 0; u < U; ++u) {
+        const int64_t pos = min(p0 + NW * u, hi - 1);  // surplus keys weigh nothing below
+        const void *kb, *vb;
+        int64_t off;
+        float ks = 1.0f, vs = 1.0f;
+        const bool from_cache = pos < pastb || p.read_all_from_cache || p.linear_cap > 0;
+        if (p.linear_cap > 0) {
+          // contiguous [batch, kv_heads, cap, head_dim] cache holding the new rows too
+          off = (((int64_t)b * p.kv_heads + kh) * p.linear_cap + pos) * Dc;
+          kb = p.key_cache;
+          vb = p.v_from_key ? p.key_cache : p.value_cache;
+        } else if (from_cache) {
+          int64_t bi = pos / p.block_size;
+          int64_t blk =
+              p.block_table[(int64_t)b * p.max_blocks + min(bi, (int64_t)p.max_blocks - 1)];
+          blk = min(max(blk, (int64_t)0), p.num_blocks - 1);
+          off = (blk * p.block_size + pos % p.block_size) * crow + (int64_t)kh * Dc;
+          kb = p.key_cache;
+          vb = p.v_from_key ? p.key_cache : p.value_cache;
+          if (std::is_same<CT, Fp8Cache>::value) {
+            ks = p.k_scale[blk * p.kv_heads + kh];
+            vs = p.v_scale[blk * p.kv_heads + kh];
+          }
+        } else {
+          int64_t tok = min(max((int64_t)s0 + (pos - pastb), (int64_t)0), (int64_t)p.num_tokens - 1);
+          off = tok * row + (int64_t)kh * D;
+          kb = p.k_new;
+          vb = p.v_from_key ? p.k_new : p.v_new;
+        }
+        part[u] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NE; ++k) {
+          const int e = lane + 64 * k;
+          vv[u][k] = 0.0f;
+          if (e < D) {
+            const float kv = from_cache
+                                 ? CacheRead<CT>::at(kb, off, e, kIntCache<CT> ? ksv[k] : ks)
+                                 : TT::to_f32(reinterpret_cast<const typename TT::raw*>(kb)[off + e]);
+            part[u] += qv[k] * kv;
+          }
+          if (e < VD)
+            vv[u][k] = from_cache
+                           ? CacheRead<CT>::at(vb, off, e, kIntCache<CT> ? vsv[k] : vs)
+                           : TT::to_f32(reinterpret_cast<const typename TT::raw*>(vb)[off + e]);
+        }
+      }
+#pragma unroll
+      for (int o2 = 32; o2 >= 1; o2 >>= 1)
+#pragma unroll
+        for (int u = 0; u < U; ++u) part[u] += __shfl_xor(part[u], o2, 64);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t pos = p0 + NW * u;
+        float s = part[u] * p.scale;
+        if (cap > 0.0f) s = cap * tanhf(s / cap);
+        if (bias_row)
+          s += TT::to_f32(
+              bias_row[min(max(min(pos, hi - 1) + bias_off, (int64_t)0), (int64_t)p.bias_cols - 1)]);
+        x[u] = pos < hi ? s * kLog2e : kNegInf;
       }
     }
-    float s = wave_sum(part) * p.scale;
-    if (cap > 0.0f) s = cap * tanhf(s / cap);
-    if (bias_row) s += TT::to_f32(bias_row[min(max(pos + bias_off, (int64_t)0), (int64_t)p.bias_cols - 1)]);
-    float x = s * kLog2e;
-    float mn = fmaxf(m, x);
-    float alpha = (m == kNegInf) ? 0.0f : exp2f(m - mn);
-    float w = exp2f(x - mn);
-    l = l * alpha + w;
+    float mn = m;
 #pragma unroll
-    for (int k = 0; k < NE; ++k) {
-      int e = lane + 64 * k;
-      if (e < VD) {
-        float vv = from_cache ? CacheRead<CT>::at(vb, off, e, kIntCache<CT> ? vsv[k] : vs)
-                              : TT::to_f32(reinterpret_cast<const typename TT::raw*>(vb)[off + e]);
-        o[k] = o[k] * alpha + w * vv;
-      }
+    for (int u = 0; u < U; ++u) mn = fmaxf(mn, x[u]);
+    // mn == -inf: every key so far weighs nothing
+    const float msafe = mn == kNegInf ? 0.0f : mn;
+    const float alpha = (m == kNegInf) ? 0.0f : exp2f(m - mn);
+    l *= alpha;
+#pragma unroll
+    for (int k = 0; k < NE; ++k) o[k] *= alpha;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float w = exp2f(x[u] - msafe);
+      l += w;
+      // (a surplus key repeats the last one's values, its weight is 0)
+#pragma unroll
+      for (int k = 0; k < NE; ++k) o[k] += w * vv[u][k];
     }
     m = mn;
+  }
+  if constexpr (NW > 1) {
+    __shared__ float wo[NW][64 * NE];
+    __shared__ float wm[NW], wl[NW];
+#pragma unroll
+    for (int k = 0; k < NE; ++k) wo[wave][lane + 64 * k] = o[k];
+    if (lane == 0) {
+      wm[wave] = m;
+      wl[wave] = l;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float mn = kNegInf;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mn = fmaxf(mn, wm[w]);
+    m = mn;
+    l = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NE; ++k) o[k] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = (wm[w] == kNegInf) ? 0.0f : exp2f(wm[w] - mn);
+      l += wl[w] * f;
+#pragma unroll
+      for (int k = 0; k < NE; ++k) o[k] += wo[w][lane + 64 * k] * f;
+    }
   }
 
   const bool single = (start == 0 && end == total);
@@ -307,25 +372,44 @@ constexpr int kMaxHeadDim = 640;
 template <int NE>
 constexpr bool ne_covers(int d) { return d <= 64 * NE; }
 
-template <typename TT, int NE>
-hipError_t launch_generic_ne(const AttnParams& p, pa_dtype cache_dtype, hipStream_t s) {
-  dim3 grid(p.max_splits, p.num_heads, p.num_tokens), block(64);
+template <typename TT, int NE, int NW>
+hipError_t launch_generic_nw(const AttnParams& p, pa_dtype cache_dtype, hipStream_t s) {
+  dim3 grid(p.max_splits, p.num_heads, p.num_tokens), block(64 * NW);
   switch (cache_dtype) {
     case PA_DTYPE_FP8_E4M3:
-      hipLaunchKernelGGL((attn_generic_kernel<TT, Fp8Cache, NE>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((attn_generic_kernel<TT, Fp8Cache, NE, NW>), grid, block, 0, s, p);
       break;
     case PA_DTYPE_INT8:
-      hipLaunchKernelGGL((attn_generic_kernel<TT, I8Cache, NE>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((attn_generic_kernel<TT, I8Cache, NE, NW>), grid, block, 0, s, p);
       break;
     case PA_DTYPE_INT4:
-      hipLaunchKernelGGL((attn_generic_kernel<TT, I4Cache, NE>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((attn_generic_kernel<TT, I4Cache, NE, NW>), grid, block, 0, s, p);
       break;
     default:
       if (cache_dtype != TT::code) return hipErrorInvalidValue;
-      hipLaunchKernelGGL((attn_generic_kernel<TT, TT, NE>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((attn_generic_kernel<TT, TT, NE, NW>), grid, block, 0, s, p);
       break;
   }
   return hipGetLastError();
+}
+
+// Wavefronts per (chunk, head, token): 16 while those workgroups fit the chip at once (512: two per
+// CU), then 4; beside at most 32 keys a workgroup holds one or two rounds at most and its meeting in
+// LDS costs more, so 4 and 1 there.  fp32, 8 heads of 64, a call with 16 / 4 / 1: one token over 2048
+// keys 21.2 / 36.4 / 109.8 us, 8 tokens over 600 22.3 / 37.0 / 110.7; 128 tokens over 128 keys 44.1 /
+// 33.2 / 83.7, 8 x 100 over 2048 1879 / 1567 / 2311; 16-token prompts 18.7 / 14.4 / 20.7 (one) and
+// 97.9 / 33.6 / 24.3 (32 of them).
+template <typename TT, int NE>
+hipError_t launch_generic_ne(const AttnParams& p, pa_dtype cache_dtype, hipStream_t s) {
+  const int64_t groups = (int64_t)p.max_splits * p.num_heads * p.num_tokens;
+  const int64_t keys =
+      p.linear_cap > 0 ? (int64_t)p.linear_cap : (int64_t)p.max_blocks * p.block_size;
+  const bool few = groups <= 512;
+  if (keys <= 32)
+    return few ? launch_generic_nw<TT, NE, 4>(p, cache_dtype, s)
+               : launch_generic_nw<TT, NE, 1>(p, cache_dtype, s);
+  return few ? launch_generic_nw<TT, NE, 16>(p, cache_dtype, s)
+             : launch_generic_nw<TT, NE, 4>(p, cache_dtype, s);
 }
 
 template <typename TT>
