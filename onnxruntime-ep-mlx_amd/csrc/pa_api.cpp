@@ -145,6 +145,10 @@ struct Plan {
   // runs on groups of sub_batch sequences in turn, the workspace sized for one group (0: the
   // whole batch in one launch).
   int sub_batch = 0;
+  // Planned prefill over images: unit list capacity; short batches in parts with fp32 partials
+  // (AttnParams::plan_fine, plan_cap slots), probabilities in two fp16 parts (plan_prec).
+  int64_t plan_units = 0, plan_cap = 0;
+  bool fine = false, prec = false;
 };
 
 // Sequences one planned launch covers.
@@ -157,9 +161,6 @@ int64_t plan_batch(const pa_batch* b, const Plan& pl) {
 // kImgMaxBytes of workspace.  PA_PREFILL_IMAGES=0 at build time keeps the in-loop conversion.
 #ifndef PA_PREFILL_IMAGES
 #define PA_PREFILL_IMAGES 1
-#endif
-#ifndef PA_IMG_WAVES
-#define PA_IMG_WAVES 2
 #endif
 constexpr int64_t kImgMinRowBlocks = 4;
 // LATENT kernel: context chunks sized for this many workgroups per CU
@@ -249,12 +250,28 @@ int latent_chunk(const pa_cache* c, const pa_batch* b, const pa_attn* a, const H
   return pick;
 }
 
+// Whether a batch of fewer items than workgroup slots runs the planned image prefill all the same
+// (given the workspace).  The plan, images and merge launches cost about 12 us more than the grid
+// launch and its reduce, so a batch of few row blocks or short contexts stays there.  A call by
+// items x longest context, planned / grid: bf16 32 heads of 128: 56 x 1200 47.0 / 38.1 us, 128 x 512
+// 42.9 / 46.9, 224 x 200 37.6 / 28.4, 224 x 1200 64.3 / 74.8, 376 x 1500 69.3 / 90.4; fp16 28 heads
+// of 128: 44 x 1200 40.1 / 35.1, 112 x 2512 55.4 / 64.0, 448 x 4048 142 / 216; fp16 24 heads of 256:
+// 96 x 512 53.4 / 61.5, 384 x 4048 272 / 542; bf16 64 heads of 64: 128 x 1064 43.8 / 43.4, 256 x 512
+// 36.2 / 51.8.
+#ifndef PA_R2_UNITS
+#define PA_R2_UNITS 96
+#endif
+bool short_planned(int64_t units, int64_t live) { return units >= PA_R2_UNITS && live >= 320; }
+
+// rich: plans that need more workspace than the plain one of the same call are allowed; run_attention
+// takes them where the caller's workspace holds them (the size queries ask for that much) and the
+// plain one otherwise.
 // images: the planned head-128 prefill may use operand images (off where the workspace is
 // bounded, pa_paged_attention_static).  bias: GroupQueryAttention's attention bias is present
 // (its streaming decode runs one wavefront per SIMD at every cache dtype).
 Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act, int kind,
                int chunk, bool linear = false, int linear_cap = 0, bool images = true,
-               bool bias = false, const HostLens& hl = HostLens()) {
+               bool bias = false, const HostLens& hl = HostLens(), bool rich = false) {
   Plan pl{};
   // The LATENT layout (values = leading dims of the key rows): its matrix-core kernel (kind 5)
   // where it covers the head sizes and dtypes, else the VALU kernel.
@@ -327,7 +344,19 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
     const int64_t rbs = ((int64_t)g * mq + pa::kPrefillRows - 1) / pa::kPrefillRows;
     const int64_t units = (int64_t)b->batch * c->kv_heads * rbs;
     const int64_t target = 2 * (int64_t)device_cus();
-    if ((units >= target || intc) && units <= (int64_t)INT32_MAX / 4 &&
+    const int64_t live_keys =
+        b->max_context_len > 0 ? std::min<int64_t>(b->max_context_len, ctx) : (int64_t)ctx;
+    // a batch of fewer items than slots, over images of rows in T (bf16 images at head 256 hold one
+    // exponent per step, where the grid kernel takes the raw values: not there)
+    const bool small = rich && PA_PREFILL_IMAGES && images && !bias && !intc && units < target &&
+                       pa::img_head(c->head_dim) &&
+                       !(act == PA_DTYPE_BFLOAT16 && c->head_dim > 128) &&
+                       pa::prefill_mfma_supported(c->head_dim, act, c->dtype) &&
+                       short_planned(units, live_keys) &&
+                       (int64_t)b->batch * c->kv_heads *
+                               ((live_keys + pa::img_keys(c->head_dim) - 1) / pa::img_keys(c->head_dim)) *
+                               pa::img_step_bytes(c->head_dim) <= kImgMaxBytes;
+    if ((units >= target || intc || small) && units <= (int64_t)INT32_MAX / 4 &&
         pa::prefill_planned_supported(c->head_dim)) {
       // Enough workgroups for every slot: planned units, longest first, long items split in two
       // (the tail of uneven row blocks otherwise idles ~28% of the slots at the C4 shape).
@@ -337,11 +366,10 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
       pl.plan_rbs = (int)rbs;
       pl.part_rows = (size_t)units * 2 * pa::kPrefillRows;
       if (PA_PREFILL_IMAGES && images && pa::img_head(c->head_dim) &&
-          (rbs >= kImgMinRowBlocks || intc)) {
+          (rbs >= kImgMinRowBlocks || intc || small)) {
         // images of the live context: the caller's bound on past + new tokens, else the capacity
         const int ik = pa::img_keys(c->head_dim);
-        const int64_t live =
-            b->max_context_len > 0 ? std::min<int64_t>(b->max_context_len, ctx) : (int64_t)ctx;
+        const int64_t live = live_keys;
         const int64_t steps = (live + ik - 1) / ik;
         const int64_t per_seq = (int64_t)c->kv_heads * steps * pa::img_step_bytes(c->head_dim);
         if ((int64_t)b->batch * per_seq <= kImgMaxBytes && steps <= 65535 &&
@@ -355,6 +383,17 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
           pl.plan_items = sub_units;
           pl.part_rows = (size_t)sub_units * 2 * pa::kPrefillRows;
         }
+      }
+      pl.plan_units = 2 * pl.plan_items;
+      if (small && pl.img_steps == 0) return make_plan(c, b, a, act, kind, 0, linear, linear_cap, images, bias, hl);
+      if (rich && units < target && pl.img_steps > 0 && pl.sub_batch == 0) {
+        // parts with fp32 partials: one slot per even share of the work and one per item
+        pl.fine = true;
+        pl.plan_cap = 2 * device_cus() + 1 + pl.plan_items;
+        pl.plan_units = std::max<int64_t>(2 * pl.plan_items, pl.plan_cap + pl.plan_items);
+        pl.part_rows = (size_t)std::max<int64_t>(2 * pl.plan_items, pl.plan_cap) * pa::kPrefillRows;
+        // the grid kernels hold the probabilities in two parts but for fp16 at head 128
+        pl.prec = small && !(act == PA_DTYPE_FLOAT16 && c->head_dim == 128);
       }
       if (!(intc && pl.img_steps == 0)) return pl;
       pl = Plan{};  // byte-coded pages whose images do not fit: see below
@@ -429,6 +468,9 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
 // Bytes of the partial rows: fp32 elements, except the planned prefill's halves, which are
 // stored as fp16 rows scaled by a power of two (store_rows with half_part).
 size_t part_o_bytes(const pa_cache* c, const Plan& pl) {
+  if (pl.fine)
+    return align256(std::max((size_t)pl.plan_items * 2 * pa::kPrefillRows * 2,
+                             (size_t)pl.plan_cap * pa::kPrefillRows * sizeof(float)) * c->head_dim);
   const size_t es = pl.plan_items > 0 ? 2 : sizeof(float);
   return align256(pl.part_rows * c->head_dim * es);
 }
@@ -437,7 +479,7 @@ size_t part_o_bytes(const pa_cache* c, const Plan& pl) {
 // Planned prefill adds [unit list (2 per item, 4 int32 each) | unit count | split flag per item].
 // Operand images add [images | step value exponents].
 size_t plan_bytes(const Plan& pl) {
-  return align256((size_t)pl.plan_items * 2 * 4 * sizeof(int32_t)) + 256 +
+  return align256((size_t)pl.plan_units * 4 * sizeof(int32_t)) + 256 +
          align256((size_t)pl.plan_items * sizeof(int32_t));
 }
 size_t image_bytes(const pa_cache* c, const pa_batch* b, const Plan& pl) {
@@ -517,13 +559,28 @@ SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_
   sp.pre_batch.max_context_len = (int32_t)std::min<int64_t>(ctx_long, INT32_MAX);
   sp.pre_batch.batch = n_long;
   sp.dec = make_plan(c, &sp.dec_batch, a, act, 0, 0, false, 0, images);
-  sp.pre = make_plan(c, &sp.pre_batch, a, act, 0, 0, false, 0, images);
+  sp.pre = make_plan(c, &sp.pre_batch, a, act, 0, 0, false, 0, images, false, HostLens(), true);
   if (!sp.dec.balanced || sp.pre.kind != 2 || sp.pre.sub_batch > 0) return sp;
   sp.seq_off = workspace_for(c, &sp.pre_batch, a, sp.pre);
   sp.bytes = std::max(workspace_for(c, &sp.dec_batch, a, sp.dec),
                       sp.seq_off + align256((size_t)n_long * sizeof(int32_t)));
   sp.on = true;
   return sp;
+}
+
+// Workspace of a call: what it needs to run, and with the plans that more workspace allows.
+struct WsNeed {
+  size_t least, best;
+};
+WsNeed ws_need(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act, int kind,
+               int chunk, bool linear = false, int linear_cap = 0, bool images = true,
+               bool bias = false, const HostLens& hl = HostLens()) {
+  WsNeed n;
+  n.least = workspace_for(
+      c, b, a, make_plan(c, b, a, act, kind, chunk, linear, linear_cap, images, bias, hl));
+  n.best = std::max(n.least, workspace_for(c, b, a, make_plan(c, b, a, act, kind, chunk, linear,
+                                                               linear_cap, images, bias, hl, true)));
+  return n;
 }
 
 // Options of one attention call beyond the public descriptors.
@@ -572,21 +629,21 @@ pa::AttnParams attn_params(const pa_cache* c, const pa_batch* b, const pa_attn* 
     char* base = reinterpret_cast<char*>(ws) + part_o_bytes(c, pl) +
                  align256(pl.part_rows * 2 * sizeof(float));
     p.plan = reinterpret_cast<int32_t*>(base);
-    base += align256((size_t)pl.plan_items * 2 * 4 * sizeof(int32_t));
+    base += align256((size_t)pl.plan_units * 4 * sizeof(int32_t));
     p.plan_info = reinterpret_cast<int32_t*>(base);
     p.plan_split = reinterpret_cast<int32_t*>(base + 256);
     p.plan_items = (int32_t)pl.plan_items;
     p.plan_rbs = pl.plan_rbs;
-    // workgroups resident per CU: two, three for the 32-key image kernel (148 VGPRs, 33 KB LDS),
-    // one for the bias kernel from head 128 on
-    p.plan_slots = (pl.img_steps > 0 && pa::img_keys(c->head_dim) == 32 && c->head_dim <= 128
-                        ? PA_IMG_WAVES
-                    : opts.bias && c->head_dim >= 128 ? 1
-                                                      : 2) * device_cus();
+    // workgroups per CU that the plan reckons with: two, one for the bias kernel from head 128 on
+    p.plan_slots = (opts.bias && c->head_dim >= 128 ? 1 : 2) * device_cus();
+    p.plan_units = (int32_t)pl.plan_units;
+    p.plan_cap = (int32_t)pl.plan_cap;
+    p.plan_fine = pl.fine ? 1 : 0;
+    p.plan_prec = pl.prec ? 1 : 0;
     p.plan_step = pl.img_steps > 0 ? pa::img_keys(c->head_dim) : pa::prefill_key_step(c->head_dim);
     if (pl.img_steps > 0) {
       const size_t hb = (size_t)plan_batch(b, pl) * c->kv_heads;
-      char* img = base + plan_bytes(pl) - align256((size_t)pl.plan_items * 2 * 4 * sizeof(int32_t));
+      char* img = base + plan_bytes(pl) - align256((size_t)pl.plan_units * 4 * sizeof(int32_t));
       p.vimg = img;
       img += align256(hb * pl.img_steps * pa::img_step_bytes(c->head_dim));
       p.vstep = reinterpret_cast<int32_t*>(img);
@@ -684,10 +741,15 @@ int run_attention(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dty
   if (opts.linear_cap > 0 && !(pl.balanced || pl.kind == 2 || pl.kind == 3))
     return fail(PA_ERR_UNSUPPORTED,
                 "contiguous caches run on the streaming decode, prefill or VALU kernels only");
-  size_t need = workspace_for(c, b, a, pl);
+  const size_t need = workspace_for(c, b, a, pl);
   if (need > 0 && (!ws || ws_bytes < need))
     return fail(PA_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes, got %zu", need,
                 ws_bytes);
+  {
+    const Plan pr = make_plan(c, b, a, act, kind, chunk, opts.linear_cap > 0, opts.linear_cap,
+                              plan_images(opts), opts.bias != nullptr, opts.host, true);
+    if (ws && ws_bytes >= workspace_for(c, b, a, pr)) pl = pr;
+  }
 
   const bool whole = kind == 0 && chunk == 0 && opts.linear_cap == 0;
   const SplitPlan sp = whole ? split_plan(c, b, a, act, opts.host, plan_images(opts)) : SplitPlan();
@@ -728,6 +790,7 @@ int run_attention(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dty
           q.block_table = p.block_table + b0 * p.max_blocks;
           q.batch = q.seqs = nb;
           q.plan_items = (int32_t)((int64_t)nb * c->kv_heads * pl.plan_rbs);
+          q.plan_units = 2 * q.plan_items;
           if (p.key_limit) q.key_limit = p.key_limit + b0;
           // fresh wide-step flags: the image slots are reused by every group
           if (b0 > 0) q.img_epoch = next_img_epoch();
@@ -942,15 +1005,14 @@ size_t pa_attention_workspace_bytes(const pa_cache* cache, const pa_batch* batch
   pa_dtype act = (cache->dtype == PA_DTYPE_FP8_E4M3 || is_int_cache(cache->dtype))
                      ? PA_DTYPE_BFLOAT16
                      : cache->dtype;
-  return workspace_for(cache, batch, attn, make_plan(cache, batch, attn, act, 0, 0));
+  return ws_need(cache, batch, attn, act, 0, 0).best;
 }
 
 size_t pa_attention_workspace_bytes_ex(const pa_cache* cache, const pa_batch* batch,
                                        const pa_attn* attn, pa_dtype act_dtype, int32_t kind,
                                        int32_t chunk_tokens) {
   if (!cache || !batch || !attn || cache->kv_heads <= 0 || batch->batch <= 0) return 0;
-  return workspace_for(cache, batch, attn,
-                       make_plan(cache, batch, attn, act_dtype, kind, chunk_tokens));
+  return ws_need(cache, batch, attn, act_dtype, kind, chunk_tokens).best;
 }
 
 int pa_attention(const pa_cache* cache, const pa_batch* batch, const pa_attn* attn,
@@ -1069,17 +1131,14 @@ int op_layout(const pa_paged_attention_node* n, const pa_paged_attention_io* io,
   a.is_causal = n->is_causal;
   a.head_sink = io->head_sink;
   a.v_head_size = L->v_head;
-  L->total = L->attn_off +
-             workspace_for(&io->cache, &b, &a,
-                           make_plan(&io->cache, &b, &a, io->dtype, 0, 0, false, 0, images,
-                                     false,
-                                     HostLens{io->host_cumulative_sequence_length,
-                                              io->host_past_seqlens}));
+  const WsNeed need = ws_need(&io->cache, &b, &a, io->dtype, 0, 0, false, 0, images, false,
+                              HostLens{io->host_cumulative_sequence_length, io->host_past_seqlens});
+  L->total = L->attn_off + need.least;
   const SplitPlan sp = split_plan(&io->cache, &b, &a, io->dtype,
                                   HostLens{io->host_cumulative_sequence_length,
                                            io->host_past_seqlens},
                                   images);
-  L->best = std::max(L->total, sp.on ? L->attn_off + sp.bytes : 0);
+  L->best = L->attn_off + std::max(need.best, sp.on ? sp.bytes : 0);
   return PA_OK;
 }
 
@@ -1339,11 +1398,10 @@ int pa_paged_attention_static(const pa_paged_attention_node* n, const pa_paged_a
 namespace {
 
 // Workspace bytes of run_attention for these descriptors and options (the same plan).
-size_t attention_ws(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act,
+WsNeed attention_ws(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act,
                     const RunOpts& o) {
-  return workspace_for(c, b, a,
-                       make_plan(c, b, a, act, 0, 0, o.linear_cap > 0, o.linear_cap,
-                                 plan_images(o), o.bias != nullptr));
+  return ws_need(c, b, a, act, 0, 0, o.linear_cap > 0, o.linear_cap, plan_images(o),
+                 o.bias != nullptr);
 }
 
 struct GqaLayout {
@@ -1357,6 +1415,7 @@ struct GqaLayout {
   bool sliding;     // sliding_window_cache: past and present are rings of capacity cap_in
   int view_cap;     // sliding: rows per (sequence, kv-head) of the staged view (cap_in + seq)
   size_t row_bytes; // bytes of one stored row of one kv-head
+  size_t best;  // as OpLayout::best
   size_t q_bytes, k_bytes, v_bytes, meta_off, pres_off, pres_side, view_off, view_side, attn_off,
       total;
   pa_cache cache;
@@ -1527,7 +1586,9 @@ int gqa_layout(const pa_gqa_node* n, const pa_gqa_io* io, GqaLayout* L) {
   o.bias_rows = io->seq;
   o.bias_cols = (int)total;
   o.smooth_softmax = n->smooth_softmax == 1;
-  L->total = L->attn_off + attention_ws(&c, &b, &a, io->dtype, o);
+  const WsNeed need = attention_ws(&c, &b, &a, io->dtype, o);
+  L->total = L->attn_off + need.least;
+  L->best = L->attn_off + need.best;
   return PA_OK;
 }
 
@@ -1604,7 +1665,7 @@ int validate_gqa_rotary(const pa_gqa_io* io) {
 size_t pa_group_query_attention_workspace_bytes(const pa_gqa_node* node, const pa_gqa_io* io) {
   GqaLayout L;
   if (gqa_layout(node, io, &L)) return 0;
-  return L.total;
+  return L.best;
 }
 
 int pa_group_query_attention(const pa_gqa_node* n, const pa_gqa_io* io, void* workspace,

@@ -1408,9 +1408,10 @@ hipError_t launch_decode_mfma(const AttnParams& p, pa_dtype act, pa_dtype cache_
 }
 
 // The partial merge of the balanced decode, for the head size of the decode launch.  Threads per
-// workgroup by the partials an average sequence has (max_splits / batch): 64 hold 4 groups of 4
-// partials in flight, 256 four times and 1024 sixteen times as many, all of an average row in one
-// round trip; more threads than that only wait on each other.
+// workgroup by the partials an average sequence can have -- max_splits / batch, at most one per
+// 32-key step of its window or block table: 64 hold 4 groups of 4 partials in flight, 256 four times
+// and 1024 sixteen times as many, all of an average row in one round trip; more threads than that
+// only wait on each other.
 template <typename TT, int D, int NT>
 void launch_merge_nt(const AttnParams& p, hipStream_t s) {
   const int rows = std::min(16, (p.num_heads / p.kv_heads) * std::max(p.max_query_len, 1));
@@ -1419,7 +1420,9 @@ void launch_merge_nt(const AttnParams& p, hipStream_t s) {
 }
 template <typename TT, int D>
 void launch_merge_d(const AttnParams& p, hipStream_t s) {
-  const int parts = p.max_splits / std::max(p.batch, 1);
+  int64_t keys = p.linear_cap > 0 ? (int64_t)p.linear_cap : (int64_t)p.max_blocks * p.block_size;
+  if (p.window > 0) keys = std::min<int64_t>(keys, (int64_t)p.window + std::max(p.max_query_len, 1));
+  const int64_t parts = std::min<int64_t>(p.max_splits / std::max(p.batch, 1), keys / 32 + 2);
   if (parts <= 8)
     launch_merge_nt<TT, D, 64>(p, s);
   else if (parts <= 64)

@@ -358,6 +358,13 @@ struct AttnParams {
   // (2 i + part - 1) * kPrefillRows + row.  plan_step: the prefill kernel's key step (32 or 64);
   // item key ranges start and split at multiples of it.
   int32_t plan_items, plan_rbs, plan_slots, plan_step;
+  // Capacity of the unit list.  plan_fine (image launches): short batches -- fewer than
+  // kPlanSplitMin keys per workgroup slot -- split their items into up to kFineParts parts with fp32
+  // partials instead, part 3 + slot of an item leaving its rows at slot * kPrefillRows; plan_cap
+  // slots.  plan_split[i] is then 2 + n + 32 * (first slot) for an item of n parts.
+  int32_t plan_units, plan_fine, plan_cap;
+  // P.V over images with the probabilities in two fp16 parts (about 22 bits)
+  int32_t plan_prec;
   // GroupQueryAttention forms (VALU kernel; the others take none of them): key_limit[b] bounds
   // the keys of sequence b (its length, below past + query rows for a ragged first prompt); bias
   // [bias_b, bias_h, bias_rows, bias_cols] in T is added to the scaled (softcapped) score of row i
@@ -394,6 +401,18 @@ struct AttnParams {
   int32_t* plan_seq;
 };
 
+// Parts of an item of a short planned prefill, at most, their keys in percent of an even share of
+// the workgroup slots (prefill_plan_kernel) and at least.
+constexpr int kFineParts = 16;
+constexpr int kFinePct = 175;
+static_assert(kFinePct >= 100, "plan_cap counts one slot per even share");
+#ifndef PA_FINE_MIN
+#define PA_FINE_MIN 256
+#endif
+// Split threshold of long planned prefills, in keys, at least (see prefill_plan_kernel).
+#ifndef PA_PLAN_SPLIT_MIN
+#define PA_PLAN_SPLIT_MIN 2048
+#endif
 // Sequences of the prefill launches of a batch split by query length, at most (the plan kernel
 // holds their list in LDS).
 constexpr int kMaxRanks = 1024;

@@ -206,7 +206,7 @@ prefill_kernel(const AttnParams p) {
   if (p.plan_items > 0) {
     // Planned: this workgroup's unit, longest first (both loads in one round trip).
     const int nunits = p.plan_info[0];
-    const int4 u = reinterpret_cast<const int4*>(p.plan)[min((int)blockIdx.x, p.plan_items * 2 - 1)];
+    const int4 u = reinterpret_cast<const int4*>(p.plan)[min((int)blockIdx.x, p.plan_units - 1)];
     if ((int)blockIdx.x >= nunits) return;
     item = u.x;
     part = u.y;
@@ -629,9 +629,15 @@ __device__ __forceinline__ void img_issue(MxBufT<KB, D>& buf, int wave, int lane
 // F8S: fp8 pages (images of the dequantised rows in fp16, keys and values each under a per-step
 // power of two): the query rows go to fp16 under a per-row power of two as for INTC, and each
 // step's key exponent joins the softmax scale of the step.
-template <typename TT, bool CAP, bool IMG, int D = 128, bool INTC = false, bool F8S = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, IMG && D <= 128 ? PA_IMG_WAVES : 2))) void
+// PREC: P.V takes the probabilities as fp16 hi + lo parts (AttnParams::plan_prec).
+// Workgroups per CU: two, bound by registers and from head 128 on by LDS; three to four at head 64
+// and up to three at 96 (33 and 49 KB of LDS).
+constexpr int mx_max_waves(bool img, int d) { return !img ? 2 : d == 64 ? 4 : d == 96 ? 3 : 2; }
+template <typename TT, bool CAP, bool IMG, int D = 128, bool INTC = false, bool F8S = false,
+          bool PREC = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, mx_max_waves(IMG, D)))) void
 prefill_mx_kernel(const AttnParams p) {
+  static_assert(!PREC || (IMG && !INTC && !F8S), "two-part probabilities over images of rows in T");
   static_assert(!(INTC || F8S) || IMG, "byte-coded pages over images only");
   using KT = typename std::conditional<INTC || F8S, TF16, TT>::type;  // score operand type
   // bf16 pages over images: steps may be wide (raw bf16 values, see kImgWideTag).  Head 256 keeps
@@ -648,7 +654,7 @@ prefill_mx_kernel(const AttnParams p) {
   int rb, kh, b, rank, split = blockIdx.y, part = 0, item = 0, ustart = 0, uend = 0;
   if (p.plan_items > 0) {
     const int nunits = p.plan_info[0];
-    const int4 u = reinterpret_cast<const int4*>(p.plan)[min((int)blockIdx.x, p.plan_items * 2 - 1)];
+    const int4 u = reinterpret_cast<const int4*>(p.plan)[min((int)blockIdx.x, p.plan_units - 1)];
     if ((int)blockIdx.x >= nunits) return;
     item = u.x;
     part = u.y;
@@ -958,7 +964,7 @@ prefill_mx_kernel(const AttnParams p) {
     }
     const float msafe = ((m_run == kNegInf) ? 0.0f : m_run) + (float)dsh;
     const _Float16 lw = (_Float16)(float)(1 << dsh);
-    u32x4 pb[2 * KB];
+    u32x4 pb[2 * KB], pl[PREC ? 2 * KB : 1];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       float pv[16];
@@ -976,13 +982,24 @@ prefill_mx_kernel(const AttnParams p) {
           pb[2 * kb + half][m] = __builtin_bit_cast(uint32_t, ph);
           // the row sum adds the fp16 probabilities the P.V product takes
           l_part = __builtin_amdgcn_fdot2(ph, f16x2v{lw, lw}, l_part, false);
+          if constexpr (PREC) {  // what fp16 left of them, rounded to fp16 once more
+            const f16x2v lo = __builtin_convertvector(
+                f32x2v{pv[8 * half + 2 * m] - (float)ph[0], pv[8 * half + 2 * m + 1] - (float)ph[1]},
+                f16x2v);
+            pl[2 * kb + half][m] = __builtin_bit_cast(uint32_t, lo);
+            l_part = __builtin_amdgcn_fdot2(lo, f16x2v{lw, lw}, l_part, false);
+          }
         }
     }
 #pragma unroll
     for (int t = 0; t < 2 * KB; ++t)
 #pragma unroll
       for (int nt = 0; nt < NQ; ++nt)
-        o[nt] = mfma32<TF16>(buf.v[t][nt][IMG ? lane : mx_vslot(lane)], pb[t], o[nt]);
+      {
+        const u32x4 vv = buf.v[t][nt][IMG ? lane : mx_vslot(lane)];
+        o[nt] = mfma32<TF16>(vv, pb[t], o[nt]);
+        if constexpr (PREC) o[nt] = mfma32<TF16>(vv, pl[t], o[nt]);
+      }
   };
   // Steps some row of this wavefront sees.
   auto seen = [&](int t0) { return t0 < any_hi && t0 + KEYS > any_lo; };
@@ -1090,9 +1107,11 @@ prefill_mx_kernel(const AttnParams p) {
         *reinterpret_cast<u32x2*>(dst + 32 * nt + 8 * i + 4 * h) = pk;
       }
     }
-  } else if (p.plan_items == 0) {
-    // split-K chunk of the grid-order launch: fp32 partial (O, m, l) for split_reduce_kernel
-    const int64_t pi = (tok * p.num_heads + head) * p.max_splits + split;
+  } else if (p.plan_items == 0 || part >= 3) {
+    // fp32 partial (O, m, l): of a split-K chunk of the grid-order launch for split_reduce_kernel, or
+    // of a part of a short planned prefill's item
+    const int64_t pi = p.plan_items == 0 ? (tok * p.num_heads + head) * p.max_splits + split
+                                         : (int64_t)(part - 3) * ROWS + (r - row0);
     float* dstf = p.part_o + pi * D;
 #pragma unroll
     for (int nt = 0; nt < NQ; ++nt)
@@ -1150,9 +1169,6 @@ prefill_mx_kernel(const AttnParams p) {
 // 55 % 342-343.
 #ifndef PA_PLAN_SPLIT_PCT
 #define PA_PLAN_SPLIT_PCT 45
-#endif
-#ifndef PA_PLAN_SPLIT_MIN
-#define PA_PLAN_SPLIT_MIN 2048
 #endif
 // Visible key range [first, end) of item i (the keys some row of the row block can see), the
 // same bounds the prefill kernel derives; end < 0 when the row block holds no rows.
@@ -1502,9 +1518,10 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
   constexpr int NB = 1024;  // buckets of 32-key steps (the last one holds everything longer)
   __shared__ int hist[NB];
   __shared__ unsigned long long total_keys;
+  __shared__ int nslots;  // fp32 partial slots given out (plan_fine)
   const int tid = threadIdx.x;
   for (int i = tid; i < NB; i += NT) hist[i] = 0;
-  if (tid == 0) total_keys = 0;
+  if (tid == 0) total_keys = 0, nslots = 0;
   // A batch split by query length: the sequences of the prefill ranks, for this kernel and, as
   // plan_seq, for the launches behind it (one wavefront, in batch order).
   __shared__ int seqs[kMaxRanks];
@@ -1550,10 +1567,38 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
   auto mid_of = [&](const ItemKeys& k) {
     return k.first + (((k.end - k.first + step - 1) / step + 1) / 2) * step;
   };
+  // A short batch (plan_fine): items in parts of at most `even` keys, kFinePct percent of a slot's
+  // even share of all keys (so plan_cap holds a slot for every share and one more per item).  More
+  // parts fill the slots more evenly but each writes and reads 128 rows of fp32 again, and a round
+  // that no longer fits the slots costs a second one.  One 512-token prompt over 2000 keys (128 items
+  // of 35 64-key steps, 512 slots): parts of 100 / 150 / 200 / 300 % take 78.4 / 69.7 / 72.2 / 71.7
+  // us a call; 320 items of 48 steps 184 / 184 / 172 / 173; 256 items at head 256 248 / 218 / 264 /
+  // 227: 175 % splits the first in three and the last in two, and leaves the second whole.
+  const bool fine = p.plan_fine && total_keys < (unsigned long long)PA_PLAN_SPLIT_MIN * p.plan_slots;
+  const int even = max(PA_FINE_MIN, (int)min(total_keys * kFinePct / (100ull * max(p.plan_slots, 1)),
+                                             (unsigned long long)INT32_MAX / 2));
+  auto steps_of = [&](const ItemKeys& k) { return (k.end - k.first + step - 1) / step; };
+  auto part_steps = [&](const ItemKeys& k) {  // key steps of each of the item's parts
+    const int s = steps_of(k), n = min((k.end - k.first + even - 1) / even, kFineParts);
+    return (s + max(n, 1) - 1) / max(n, 1);
+  };
   for (int i = tid, j = 0; i < p.plan_items; i += NT, ++j) {
     const ItemKeys k = keys(j, i);
     if (k.end < 0) {
       p.plan_split[i] = 0;
+      continue;
+    }
+    if (fine) {
+      const int s = steps_of(k), per = part_steps(k), n = per > 0 ? (s + per - 1) / per : 1;
+      const int base = n > 1 ? atomicAdd(&nslots, n) : 0;
+      const bool sp = n > 1 && base + n <= p.plan_cap;
+      p.plan_split[i] = sp ? 2 + n + 32 * base : 0;
+      if (sp) {
+        for (int u = 0; u < n; ++u)
+          atomicAdd(&hist[bucket(min(k.first + (u + 1) * per * step, k.end) - (k.first + u * per * step))], 1);
+      } else {
+        atomicAdd(&hist[bucket(k.end - k.first)], 1);
+      }
       continue;
     }
     const bool sp = split_of(k);
@@ -1599,6 +1644,19 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
   for (int i = tid, j = 0; i < p.plan_items; i += NT, ++j) {
     const ItemKeys k = keys(j, i);
     if (k.end < 0) continue;
+    if (fine) {
+      const int v = p.plan_split[i];  // this thread's own store above
+      if (v == 0) {
+        plan[atomicAdd(&hist[bucket(k.end - k.first)], 1)] = int4{i, 0, k.first, k.end};
+      } else {
+        const int n = (v - 2) & 31, base = (v - 2) >> 5, per = part_steps(k);
+        for (int u = 0; u < n; ++u) {
+          const int a = k.first + u * per * step, e = min(a + per * step, k.end);
+          plan[atomicAdd(&hist[bucket(e - a)], 1)] = int4{i, 3 + base + u, a, e};
+        }
+      }
+      continue;
+    }
     if (split_of(k)) {
       const int mid = mid_of(k);
       plan[atomicAdd(&hist[bucket(mid - k.first)], 1)] = int4{i, 1, k.first, mid};
@@ -1629,7 +1687,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p) 
   static_assert(kPrefillRows % kPrefillMergeRows == 0 && kPrefillMergeRows % RPP == 0, "merge tiling");
   constexpr int CH = kPrefillRows / kPrefillMergeRows;
   const int i = blockIdx.x / CH;
-  if (!p.plan_split[i]) return;
+  const int form = p.plan_split[i];
+  if (!form) return;
   const int g = p.num_heads / p.kv_heads;
   const int kh = i % p.kv_heads, rb = (i / p.kv_heads) % p.plan_rbs;
   int b = i / (p.kv_heads * p.plan_rbs);
@@ -1640,6 +1699,63 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p) 
   // Every load in one round trip: the sequence bounds, both halves' (m, l) and rows, the sink.
   // Rows past the block's last row read in-bounds workspace rows and store nothing.
   const int cb0 = p.cum[b], cb1 = p.cum[b + 1];
+  if (form > 1) {
+    // fp32 parts of a short batch's item, kMergeParts of them in flight per row
+    constexpr int kMergeParts = 4;
+    const int n = (form - 2) & 31, base = (form - 2) >> 5;
+    const int t0 = min(max(cb0, 0), p.num_tokens), t1 = min(max(cb1, t0), p.num_tokens);
+    const int nrows = min(kPrefillRows, g * (t1 - t0) - row0);
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const int r = rbase + j * RPP;
+      if (r >= nrows) continue;
+      const int rr = row0 + r, h = kh * g + rr % g;
+      const int64_t t = t0 + rr / g;
+      const float sink = sink_logit<TT>(p, h);
+      float M = kNegInf, L = 0.0f;
+      f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
+      for (int k0 = 0; k0 < n; k0 += kMergeParts) {
+        float2 ml[kMergeParts];
+        f32x4 v0[kMergeParts], v1[kMergeParts];
+#pragma unroll
+        for (int u = 0; u < kMergeParts; ++u) {
+          const int64_t row = (int64_t)(base + min(k0 + u, n - 1)) * kPrefillRows + r;
+          ml[u] = reinterpret_cast<const float2*>(p.part_ml)[row];
+          const f32x4* src = reinterpret_cast<const f32x4*>(p.part_o + row * D + 8 * q);
+          v0[u] = src[0];
+          v1[u] = src[1];
+        }
+        float mn = M;
+#pragma unroll
+        for (int u = 0; u < kMergeParts; ++u)
+          if (k0 + u < n) mn = fmaxf(mn, ml[u].x);
+        const float a = (M == kNegInf) ? 0.0f : exp2f(M - mn);
+        L *= a;
+        x0 *= a;
+        x1 *= a;
+#pragma unroll
+        for (int u = 0; u < kMergeParts; ++u) {
+          const float w = (k0 + u < n && ml[u].x != kNegInf) ? exp2f(ml[u].x - mn) : 0.0f;
+          L += ml[u].y * w;
+          if (w != 0.0f) {
+            x0 += v0[u] * w;
+            x1 += v1[u] * w;
+          }
+        }
+        M = mn;
+      }
+      const float f = finalize_factor(M, L, sink);
+      u32x4 pk;
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        pk[m] = (uint32_t)TT::from_f32(x0[2 * m] * f) | ((uint32_t)TT::from_f32(x0[2 * m + 1] * f) << 16);
+        pk[2 + m] = (uint32_t)TT::from_f32(x1[2 * m] * f) | ((uint32_t)TT::from_f32(x1[2 * m + 1] * f) << 16);
+      }
+      *reinterpret_cast<u32x4*>(reinterpret_cast<typename TT::raw*>(p.out) +
+                                (t * p.num_heads + h) * D + 8 * q) = pk;
+    }
+    return;
+  }
   float2 a[NP], c[NP];
   u32x4 ha[NP], hc[NP];  // fp16 partial rows (store_rows, half_part)
   float sk[NP];
@@ -1710,6 +1826,11 @@ hipError_t launch_d(const AttnParams& p, dim3 grid, hipStream_t s, int pk = kPkT
           hipLaunchKernelGGL((prefill_mx_kernel<TT, true, true, D, false, true>), grid, dim3(256), 0, s, p);
         else
           hipLaunchKernelGGL((prefill_mx_kernel<TT, false, true, D, false, true>), grid, dim3(256), 0, s, p);
+      } else if (p.plan_prec) {
+        if (p.softcap > 0.0f)
+          hipLaunchKernelGGL((prefill_mx_kernel<TT, true, true, D, false, false, true>), grid, dim3(256), 0, s, p);
+        else
+          hipLaunchKernelGGL((prefill_mx_kernel<TT, false, true, D, false, false, true>), grid, dim3(256), 0, s, p);
       } else if (p.softcap > 0.0f) {
         hipLaunchKernelGGL((prefill_mx_kernel<TT, true, true, D>), grid, dim3(256), 0, s, p);
       } else {
@@ -1781,6 +1902,7 @@ hipError_t launch_prefill_planned(const AttnParams& p, pa_dtype act, pa_dtype ca
       !p.plan_split || !p.part_o || !p.part_ml || p.max_splits != 1)
     return hipErrorInvalidValue;
   if ((int64_t)p.plan_items * (kPrefillRows / kPrefillMergeRows) > INT32_MAX) return hipErrorInvalidValue;
+  if (p.plan_units < 2 * p.plan_items || (p.plan_fine && !p.vimg)) return hipErrorInvalidValue;
   if (p.seqs < 1 || (p.short_tokens > 0 && (!p.plan_seq || p.seqs > kMaxRanks)))
     return hipErrorInvalidValue;
   // Operand images: written by workgroups 1.. of the plan launch.
@@ -1826,7 +1948,7 @@ hipError_t launch_prefill_planned(const AttnParams& p, pa_dtype act, pa_dtype ca
     else
       by_head(TBF16{});
   }
-  const dim3 grid(2 * p.plan_items, 1);
+  const dim3 grid(p.plan_units, 1);
   hipError_t e = act == PA_DTYPE_FLOAT16 ? launch_t<TF16>(p, grid, s, pk)
                                          : launch_t<TBF16>(p, grid, s, pk);
   if (e != hipSuccess) return e;
