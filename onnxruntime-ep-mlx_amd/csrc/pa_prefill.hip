@@ -1508,7 +1508,8 @@ __device__ __forceinline__ void image_steps(const AttnParams& p, int id) {
 }
 
 template <int NT, typename TT, int IMGD, int KC = kImgT>
-__global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
+// (at most 64 VGPRs: two image workgroups of 1024 threads per CU; one cost half the image rate)
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void prefill_plan_kernel(const AttnParams p) {
   if constexpr (IMGD > 0) {  // head size of the operand images; KC: the pages' element kind
     if (blockIdx.x > 0) {
       image_steps<TT, NT, IMGD, KC>(p, (int)blockIdx.x - 1);
@@ -1539,18 +1540,26 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
   }
   __syncthreads();
   // The key ranges of this thread's first kCached items stay in registers for the later passes
-  // (each costs two dependent metadata loads).
+  // (each costs two dependent metadata loads); unrolled, since an indexed array would be kept in LDS
+  // (32 KB) or scratch.
   constexpr int kCached = 4;
   ItemKeys cached[kCached];
-  auto keys = [&](int j, int i) { return j < kCached ? cached[j] : item_keys(p, i, seqs); };
   unsigned long long mine = 0;
-  for (int i = tid, j = 0; i < p.plan_items; i += NT, ++j) {
-    const ItemKeys k = item_keys(p, i, seqs);
 #pragma unroll
-    for (int c = 0; c < kCached; ++c)
-      if (c == j) cached[c] = k;
+  for (int j = 0; j < kCached; ++j) {
+    cached[j] = tid + j * NT < p.plan_items ? item_keys(p, tid + j * NT, seqs) : ItemKeys{0, -1};
+    if (cached[j].end >= 0) mine += (unsigned long long)(cached[j].end - cached[j].first);
+  }
+  for (int i = tid + kCached * NT; i < p.plan_items; i += NT) {
+    const ItemKeys k = item_keys(p, i, seqs);
     if (k.end >= 0) mine += (unsigned long long)(k.end - k.first);
   }
+  auto each = [&](auto&& take) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kCached; ++j)
+      if (tid + j * NT < p.plan_items) take(tid + j * NT, cached[j]);
+    for (int i = tid + kCached * NT; i < p.plan_items; i += NT) take(i, item_keys(p, i, seqs));
+  };
   // Wave sums first: one LDS atomic per wavefront instead of one per thread on one address.
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) mine += __shfl_xor(mine, o, 64);
@@ -1582,11 +1591,10 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
     const int s = steps_of(k), n = min((k.end - k.first + even - 1) / even, kFineParts);
     return (s + max(n, 1) - 1) / max(n, 1);
   };
-  for (int i = tid, j = 0; i < p.plan_items; i += NT, ++j) {
-    const ItemKeys k = keys(j, i);
+  each([&](int i, const ItemKeys& k) __attribute__((always_inline)) {
     if (k.end < 0) {
       p.plan_split[i] = 0;
-      continue;
+      return;
     }
     if (fine) {
       const int s = steps_of(k), per = part_steps(k), n = per > 0 ? (s + per - 1) / per : 1;
@@ -1599,7 +1607,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
       } else {
         atomicAdd(&hist[bucket(k.end - k.first)], 1);
       }
-      continue;
+      return;
     }
     const bool sp = split_of(k);
     p.plan_split[i] = sp ? 1 : 0;
@@ -1610,7 +1618,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
     } else {
       atomicAdd(&hist[bucket(k.end - k.first)], 1);
     }
-  }
+  });
   __syncthreads();
   {  // exclusive scan of the histogram, one bucket per thread: wave scans, then the wave sums
     static_assert(NT == NB && NT % 64 == 0 && NT / 64 <= 64, "one bucket per thread");
@@ -1641,9 +1649,8 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
   }
   __syncthreads();
   int4* plan = reinterpret_cast<int4*>(p.plan);
-  for (int i = tid, j = 0; i < p.plan_items; i += NT, ++j) {
-    const ItemKeys k = keys(j, i);
-    if (k.end < 0) continue;
+  each([&](int i, const ItemKeys& k) __attribute__((always_inline)) {
+    if (k.end < 0) return;
     if (fine) {
       const int v = p.plan_split[i];  // this thread's own store above
       if (v == 0) {
@@ -1655,7 +1662,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
           plan[atomicAdd(&hist[bucket(e - a)], 1)] = int4{i, 3 + base + u, a, e};
         }
       }
-      continue;
+      return;
     }
     if (split_of(k)) {
       const int mid = mid_of(k);
@@ -1664,7 +1671,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(const AttnParams p) {
     } else {
       plan[atomicAdd(&hist[bucket(k.end - k.first)], 1)] = int4{i, 0, k.first, k.end};
     }
-  }
+  });
 }
 
 // Merge the two halves of each split item: one workgroup per kPrefillMergeRows rows of an
