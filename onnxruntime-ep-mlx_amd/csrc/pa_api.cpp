@@ -517,16 +517,18 @@ struct SplitPlan {
   size_t seq_off = 0, bytes = 0;  // list of the prefill sequences, workspace in all
 };
 
-// Key/value bytes (as 16-bit rows) of the decode sequences from which a batch is split.  One launch
-// for all of them takes the planned prefill with fewer long rows than the long sequences alone need
-// for it, so small decode shares stay with it: with one prompt of 64 / 512 / 1500 tokens beside 48
-// contexts of 1000 (197 MB at 8 kv-heads of 128) 64.2 / 91.5 / 137.8 us split, 56.2 / 154.0 / 197.7
-// whole, 32 of 2000 (262 MB) 73.2 / 98.3 / 150.7 against 87.7 / 201.1 / 217.9; at head 256 48 of
-// 1000 beside 1500 tokens 238.7 against 215.4, 32 of 2000 230.7 against 257.9.  48 contexts of up
-// to 6000 and three prompts of up to 600 tokens: 390 -> 210 us a call.
-#ifndef PA_SPLIT_MIN_BYTES
-#define PA_SPLIT_MIN_BYTES (224ll << 20)
-#endif
+// Key/value bytes (as 16-bit rows) of the decode sequences from which a batch is split.  The split
+// costs the decode's two launches, and few long rows lose the planned launch that all rows together
+// fill; what it saves grows with the decode sequences' contexts.  One prompt of 64 / 300 / 1500 tokens
+// beside them, bf16, 8 kv-heads of 128, split against whole: 16 contexts of 500 (33 MB) 37.6 / 59.3 /
+// 92.3 against 40.2 / 50.2 / 88.2 us, 8 of 2000 (66 MB) 44.1 / 56.1 / 98.5 against 56.4 / 89.3 /
+// 103.2, 16 of 2000 53.4 / 65.2 / 108.5 against 91.7 / 121.3 / 140.3; fp16, head 256, 8 of 2000 51.1 /
+// 82.5 / 122.4 against 60.6 / 123.0 / 137.2.  bf16 prompts at head 256 keep to the grid kernel below
+// 512 row blocks: 48 contexts of 1000 (197 MB) beside 1500 tokens 239.4 against 216.0, 32 of 2000
+// 230.7 against 257.9.
+int64_t split_min_bytes(const pa_cache* c, pa_dtype act) {
+  return (int64_t)(act == PA_DTYPE_BFLOAT16 && c->head_dim > 128 ? 224 : 60) << 20;
+}
 
 SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act,
                      const HostLens& hl, bool images) {
@@ -550,7 +552,7 @@ SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_
     }
   }
   if (n_long == 0 || n_long > pa::kMaxRanks || mq_short == 0 ||
-      keys * c->kv_heads * c->head_dim * 4 < (int64_t)PA_SPLIT_MIN_BYTES)
+      keys * c->kv_heads * c->head_dim * 4 < split_min_bytes(c, act))
     return sp;
   sp.short_tokens = limit;
   sp.dec_batch = sp.pre_batch = *b;

@@ -117,7 +117,7 @@ class Mixed:
 
 
 # heads, kv, head, block, new tokens, past: the decode sequences hold 240 MB and more of 16-bit keys
-# and values, the others fill the grid launch or (more rows) the planned one
+# and values (the last two 64 to 70), the others run the grid launch or (more rows) the planned one
 SHAPES = [
     (32, 8, 128, 16, [1, 1, 40, 1, 0, 2, 1, 300], [13900, 16201, 33, 15640, 50, 777, 15500, 0]),
     (16, 2, 64, 16, [1] * 70 + [513, 1, 129], [6800] * 70 + [64, 1, 2000]),  # ranks past 64
@@ -125,6 +125,8 @@ SHAPES = [
     (8, 4, 96, 16, [700, 1, 1, 900, 1], [0, 82500, 81801, 300, 2000]),
     (28, 4, 128, 16, [2, 1, 513, 600, 512, 64, 1], [61000, 62999, 700, 0, 1300, 5, 1]),
     (64, 8, 64, 16, [1000, 900, 800, 1, 1], [0, 10, 500, 63100, 61000]),
+    (32, 8, 128, 16, [1] * 20 + [400], [800] * 20 + [3]),
+    (24, 4, 256, 256, [1, 130, 2, 1], [5000, 900, 5300, 5200]),
 ]
 FORMS = [dict(rot=32), dict(dtype="float16", window=31000, softcap=20.0, sink=True)]
 
