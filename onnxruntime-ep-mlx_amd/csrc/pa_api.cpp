@@ -215,6 +215,9 @@ struct HostLens {
 #ifndef PA_LATENT_ODD_SPLITS
 #define PA_LATENT_ODD_SPLITS 1
 #endif
+#ifndef PA_LATENT_WIDE_ROWS
+#define PA_LATENT_WIDE_ROWS 16
+#endif
 constexpr int kLatPlanMaxBatch = 4096;  // batches beyond this keep the capacity rule (host cost)
 
 // LATENT kernel: the context chunk (a multiple of 32 keys in [256, cap]) that minimises the
@@ -226,28 +229,57 @@ int latent_chunk(const pa_cache* c, const pa_batch* b, const pa_attn* a, const H
                  int ng, int64_t slots, int cap) {
   const int D = c->head_dim;
   const int64_t H = a->num_heads;
+  // Per sequence its keys, row blocks and rows, once; a candidate then takes one division a sequence,
+  // in double (whole numbers this small give the exact floor), where three 64-bit ones each made the
+  // search over 64 sequences 25 us of host time
+  std::vector<double> seqs((size_t)3 * std::max(b->batch, 0));
+  double *keys = seqs.data(), *blocks = keys + b->batch, *rows = blocks + b->batch;
+  int m = 0;
+  double steps = 0.0;
+  for (int i = 0; i < b->batch; ++i) {
+    const int64_t nq = (int64_t)hl.cum[i + 1] - hl.cum[i];
+    if (nq <= 0) continue;
+    const int64_t tot = std::max<int64_t>((int64_t)std::max(hl.past[i], 0) + nq, 1);
+    const int64_t rbs = (H * nq + 16 * ng - 1) / (16 * ng);
+    steps += (double)(rbs * ((tot + 31) / 32));
+    keys[m] = (double)tot;
+    blocks[m] = (double)rbs;
+    rows[m++] = (double)(H * nq);
+  }
   double best = 0.0;
   int pick = 0;
   for (int ch = 256; ch <= cap; ch += 32) {
-    int64_t work = 0, part_rows = 0;
-    for (int i = 0; i < b->batch; ++i) {
-      const int64_t nq = (int64_t)hl.cum[i + 1] - hl.cum[i];
-      if (nq <= 0) continue;
-      const int64_t tot = std::max<int64_t>((int64_t)std::max(hl.past[i], 0) + nq, 1);
-      const int64_t rbs = (H * nq + 16 * ng - 1) / (16 * ng);
-      const int64_t n = (tot + ch - 1) / ch;
-      work += rbs * ((tot + 31) / 32 + n);  // steps + one step of set-up per workgroup
-      if (n > 1) part_rows += n * H * nq;
+    double work = steps, part_rows = 0.0;
+    for (int i = 0; i < m; ++i) {
+      const double n = (double)(int32_t)((keys[i] + (ch - 1)) / ch);
+      work += blocks[i] * n;  // one step of set-up per workgroup
+      part_rows += n > 1.0 ? n * rows[i] : 0.0;
     }
     const double merge =
-        PA_LATENT_MERGE_W * (double)part_rows * (D * 4 + 8) * 2 / ((double)slots * 32 * D * 2);
-    const double est = (double)work / (double)slots + (ch / 32 + 1) * 0.5 + merge;
+        PA_LATENT_MERGE_W * part_rows * (D * 4 + 8) * 2 / ((double)slots * 32 * D * 2);
+    const double est = work / (double)slots + (ch / 32 + 1) * 0.5 + merge;
     if (pick == 0 || est < best) {
       best = est;
       pick = ch;
     }
   }
   return pick;
+}
+
+// MLA batches that run in 64-row blocks (kind 6) given the workspace: from 16 grouped query rows, of
+// where most products run on padding: each row still leaves HBM once, and the segments fill the chip
+// whatever the contexts.  A call, 64-row blocks against the 16- and 32-row ones, contexts of
+// 200 .. 300 / 1333 .. 2000 / 2667 .. 4000 keys: 16 heads, 4 sequences 21.0 / 23.0 against 31.5 / 31.4
+// us, 32 of them 24.9 / 39.3 against 32.3 / 36.2, 64 33.6 / - / 78.3 against 36.4 / - / 109; 64 heads,
+// 4 sequences 25.7 / 33.8 against 43.0 / 39.7, 64 47.6 / - / 98.4 against 46.6 / - / 223; 128 heads, 16
+// sequences 37.0 / 55.7 against 45.0 / 93.2, 64 58.0 / - / 147 against 51.4 / - / 371; prompts, 128 heads
+// of 100 tokens after 1000 93 against 201, two of 256 after 2000 526 against 1404.
+bool latent_wide(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act) {
+  const int mq = b->max_query_len > 0 ? b->max_query_len : std::max(b->num_tokens, 1);
+  return (int64_t)a->num_heads * mq >= PA_LATENT_WIDE_ROWS &&
+         pa::latent_wide_supported(c->head_dim, a->v_head_size, act, c->dtype, c->block_size,
+                                   b->max_blocks, b->batch,
+                                   pa::latent_wide_row_blocks(a->num_heads, mq));
 }
 
 // Whether a batch of fewer items than workgroup slots runs the planned image prefill all the same
@@ -284,6 +316,13 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
   }
   const int g = a->num_heads / c->kv_heads;
   const int mq = b->max_query_len > 0 ? b->max_query_len : std::max(b->num_tokens, 1);
+  if (kind == 5 && rich && chunk <= 0 && latent_wide(c, b, a, act)) {
+    pl.kind = 6;
+    pl.chunk = 32;
+    pl.max_splits = device_cus();
+    pl.part_rows = (size_t)2 * pl.max_splits * pa::kLatWideRows;
+    return pl;
+  }
   const bool mfma = pa::decode_mfma_supported(c->head_dim, act, c->dtype);
   // The balanced (streaming) decode addresses rows with 32-bit row indices and shifts, and
   // numbers the 32-key steps of the whole batch with 32-bit indices: every sequence is clamped
@@ -472,7 +511,7 @@ size_t part_o_bytes(const pa_cache* c, const Plan& pl) {
     return align256(std::max((size_t)pl.plan_items * 2 * pa::kPrefillRows * 2,
                              (size_t)pl.plan_cap * pa::kPrefillRows * sizeof(float)) * c->head_dim);
   const size_t es = pl.plan_items > 0 ? 2 : sizeof(float);
-  return align256(pl.part_rows * c->head_dim * es);
+  return align256(pl.part_rows * (pl.kind == 6 ? pa::kLatWideDims : c->head_dim) * es);
 }
 
 // Workspace: [partial O | partial (m, l)].
@@ -501,6 +540,7 @@ size_t workspace_for(const pa_cache* c, const pa_batch* b, const pa_attn*, const
   if (pl.part_rows == 0) return 0;
   size_t n = part_o_bytes(c, pl) + align256(pl.part_rows * 2 * sizeof(float));
   if (pl.plan_items > 0) n += plan_bytes(pl) + image_bytes(c, b, pl);
+  if (pl.kind == 6) n += align256((size_t)pl.max_splits * 4 * sizeof(int32_t));
   return n;
 }
 
@@ -570,6 +610,12 @@ SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_
   return sp;
 }
 
+// Whether a call whose plain plan is pl has no richer one (and the search for pl's chunk need not run
+// again to find that out).
+bool plain_only(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act, const Plan& pl) {
+  return pl.kind != 2 && !(pl.kind == 5 && latent_wide(c, b, a, act));
+}
+
 // Workspace of a call: what it needs to run, and with the plans that more workspace allows.
 struct WsNeed {
   size_t least, best;
@@ -578,8 +624,9 @@ WsNeed ws_need(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
                int chunk, bool linear = false, int linear_cap = 0, bool images = true,
                bool bias = false, const HostLens& hl = HostLens()) {
   WsNeed n;
-  n.least = workspace_for(
-      c, b, a, make_plan(c, b, a, act, kind, chunk, linear, linear_cap, images, bias, hl));
+  const Plan plain = make_plan(c, b, a, act, kind, chunk, linear, linear_cap, images, bias, hl);
+  n.best = n.least = workspace_for(c, b, a, plain);
+  if (plain_only(c, b, a, act, plain)) return n;
   n.best = std::max(n.least, workspace_for(c, b, a, make_plan(c, b, a, act, kind, chunk, linear,
                                                                linear_cap, images, bias, hl, true)));
   return n;
@@ -627,6 +674,9 @@ pa::AttnParams attn_params(const pa_cache* c, const pa_batch* b, const pa_attn* 
   p.part_o = need ? reinterpret_cast<float*>(ws) : nullptr;
   p.part_ml = need ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + part_o_bytes(c, pl))
                    : nullptr;
+  if (pl.kind == 6)
+    p.plan_info = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(ws) + part_o_bytes(c, pl) +
+                                             align256(pl.part_rows * 2 * sizeof(float)));
   if (pl.plan_items > 0) {
     char* base = reinterpret_cast<char*>(ws) + part_o_bytes(c, pl) +
                  align256(pl.part_rows * 2 * sizeof(float));
@@ -747,10 +797,13 @@ int run_attention(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dty
   if (need > 0 && (!ws || ws_bytes < need))
     return fail(PA_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes, got %zu", need,
                 ws_bytes);
-  {
+  if (!plain_only(c, b, a, act, pl)) {
     const Plan pr = make_plan(c, b, a, act, kind, chunk, opts.linear_cap > 0, opts.linear_cap,
                               plan_images(opts), opts.bias != nullptr, opts.host, true);
-    if (ws && ws_bytes >= workspace_for(c, b, a, pr)) pl = pr;
+    // (the wide LATENT kernel reads every row from the pages)
+    const bool paged = opts.new_rows_in_cache ||
+                       ((b->flags & PA_BATCH_NEW_ROWS_IN_CACHE) && !b->slot_mapping);
+    if (ws && ws_bytes >= workspace_for(c, b, a, pr) && (pr.kind != 6 || paged)) pl = pr;
   }
 
   const bool whole = kind == 0 && chunk == 0 && opts.linear_cap == 0;
@@ -775,6 +828,11 @@ int run_attention(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dty
   if (pl.balanced) {
     e = pa::launch_decode_balanced(p, act, c->dtype, s);  // attention + partial merge
     if (e != hipSuccess) return hip_fail(e, "balanced decode launch");
+    return PA_OK;
+  }
+  if (pl.kind == 6) {
+    e = pa::launch_latent_wide(p, act, c->dtype, s);  // attention + partial merge
+    if (e != hipSuccess) return hip_fail(e, "LATENT kernel launch");
     return PA_OK;
   }
   switch (pl.kind) {

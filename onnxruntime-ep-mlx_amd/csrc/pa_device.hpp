@@ -538,6 +538,16 @@ bool latent_mfma_supported(int head_dim, int v_head_dim, pa_dtype act, pa_dtype 
 // 16-row groups per LATENT workgroup for H heads and max_query_len mq.
 inline int latent_row_groups(int heads, int mq) { return (int64_t)heads * mq >= 32 ? 2 : 1; }
 hipError_t launch_latent(const AttnParams& p, pa_dtype act, pa_dtype cache_dtype, hipStream_t s);
+// MLA rows against blocks of 64 grouped query rows (pa_latent.hip); max_splits: its workgroups, each
+// with two partial slots of kLatWideRows rows of kLatWideDims.
+constexpr int kLatWideRows = 64, kLatWideDims = 512;
+bool latent_wide_supported(int head_dim, int v_head_dim, pa_dtype act, pa_dtype cache_dtype,
+                           int block_size, int max_blocks, int batch, int64_t rbs);
+inline int64_t latent_wide_row_blocks(int heads, int mq) {
+  return ((int64_t)heads * mq + kLatWideRows - 1) / kLatWideRows;
+}
+hipError_t launch_latent_wide(const AttnParams& p, pa_dtype act, pa_dtype cache_dtype,
+                              hipStream_t s);
 // GroupQueryAttention output_qk diagnostics (pa_attn_generic.hip): mode 1 scores, 2 probabilities
 // into qk [batch, num_heads, max_query_len, cols]; keys[b]: the sequence's key count.
 hipError_t launch_gqa_qk(const AttnParams& p, pa_dtype act, pa_dtype cache_dtype, void* qk,
