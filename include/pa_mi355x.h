@@ -177,7 +177,8 @@ int pa_rotary_append(const pa_cache* cache, const pa_batch* batch, int32_t num_h
 int pa_reshape_and_cache(const pa_cache* cache, const pa_batch* batch, pa_dtype act_dtype,
                          const void* key, const void* value, pa_stream_t stream);
 
-/* Workspace (bytes) needed by pa_attention for split-K partials. */
+/* Workspace (bytes) that pa_attention can use for its partials, plans and images.  A call also runs
+ * with less, down to what the plainest plan of its shapes needs (below that: "workspace too small"). */
 size_t pa_attention_workspace_bytes(const pa_cache* cache, const pa_batch* batch,
                                     const pa_attn* attn);
 /* Workspace (bytes) needed by pa_attention_ex for the given kind / chunk. */
@@ -198,14 +199,16 @@ size_t pa_attention_workspace_bytes_ex(const pa_cache* cache, const pa_batch* ba
  *   - other batches over pages in T: the LDS-shared prefill kernel (128 grouped query rows per
  *     workgroup; the planned launch -- longest-first units, long items split in two -- once the
  *     batch fills two workgroups per compute unit, over operand images when each (sequence,
- *     kv-head) has at least 4 row blocks);
+ *     kv-head) has at least 4 row blocks; also from 96 such row blocks and 320 live keys on with the
+ *     queried workspace, except bf16 at head 256);
  *   - other batches over fp8 / int8 / int4 pages: the planned prefill over operand images (fp16
  *     rows of the live context, within 2 GiB of workspace; larger batches run it on groups of
  *     sequences whose images fit, one launch per group);
  *   - the LATENT layout (one kv-head, values = the first v_head_size key dims) with the cache in
  *     the activation dtype, key rows of a multiple of 32 dims up to 640 and values of 128, 256
- *     or 512 dims (MLA 576 / 512): its matrix-core kernel, all heads served by one read of each
- *     row per 16 grouped query rows;
+ *     or 512 dims (MLA 576 / 512): its matrix-core kernels, all heads served by one read of each
+ *     row per 16 or 32 grouped query rows, and per 64 at 576 / 512 with 16 or more of them, the new
+ *     rows in the pages, whole 16-row tiles per page and the queried workspace;
  *   - fp32 activations, other head sizes, other LATENT shapes and forced split-K chunks over
  *     byte-coded pages: the VALU kernel.
  * batch->max_query_len = 0 is read as num_tokens. */
