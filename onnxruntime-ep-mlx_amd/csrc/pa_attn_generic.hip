@@ -222,9 +222,11 @@ __global__ __launch_bounds__(64 * NW) void attn_generic_kernel(const AttnParams 
     for (int u = 0; u < U; ++u) {
       const float w = exp2f(x[u] - msafe);
       l += w;
-      // (a surplus key repeats the last one's values, its weight is 0)
+      // a surplus key repeats the row's last one: weight 0, and its values, which may be infinite, left
+      // out (the test is the same for the whole wavefront)
+      if (u == 0 || p0 + NW * u < hi)
 #pragma unroll
-      for (int k = 0; k < NE; ++k) o[k] += w * vv[u][k];
+        for (int k = 0; k < NE; ++k) o[k] += w * vv[u][k];
     }
     m = mn;
   }
