@@ -1256,8 +1256,9 @@ __global__ __launch_bounds__(NT) void balanced_merge_kernel(const AttnParams p) 
     for (int j = 0; j < kMergeDepth; ++j) {
       const float w = (k0 + j * PG < nparts && ml[j].x != kNegInf) ? exp2f(ml[j].x - mn) : 0.0f;
       lsum += ml[j].y * w;
-      // a surplus piece's row may hold anything in a piece that saw no key: not multiplied in
-      if (w != 0.0f) acc += o[j] * w;
+      // Surplus loads are left out (a piece again, maybe infinite); every piece counts, also one of
+      // weight 0, whose row is NaN where its scores are
+      if (k0 + j * PG < nparts) acc += o[j] * w;
     }
     M = mn;
   }

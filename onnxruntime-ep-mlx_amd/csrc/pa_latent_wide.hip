@@ -472,7 +472,7 @@ __global__ __launch_bounds__(128 * GR) void latent_merge_kernel(const AttnParams
   auto add = [&](float m, float l, f32x4 v, float mn) {
     const float wt = m != kNegInf ? exp2f(m - mn) : 0.0f;
     lsum += l * wt;
-    if (wt != 0.0f) acc += v * wt;
+    acc += v * wt;  // also at weight 0: the row is NaN where the partial's scores are
   };
   for (int k0 = gr; k0 < nparts; k0 += U * GR) {
     float2 ml[U];

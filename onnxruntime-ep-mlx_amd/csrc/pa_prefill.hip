@@ -1744,7 +1744,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p) 
         for (int u = 0; u < kMergeParts; ++u) {
           const float w = (k0 + u < n && ml[u].x != kNegInf) ? exp2f(ml[u].x - mn) : 0.0f;
           L += ml[u].y * w;
-          if (w != 0.0f) {
+          if (k0 + u < n) {  // every part, also of weight 0 (NaN where its scores are); no surplus load
             x0 += v0[u] * w;
             x1 += v1[u] * w;
           }
