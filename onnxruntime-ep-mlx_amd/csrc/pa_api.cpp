@@ -146,7 +146,7 @@ struct Plan {
   // whole batch in one launch).
   int sub_batch = 0;
   // Planned prefill over images: unit list capacity; short batches in parts with fp32 partials
-  // (AttnParams::plan_fine, plan_cap slots), probabilities in two fp16 parts (plan_prec).
+  // (AttnParams::plan_fine, plan_cap slots), probabilities in two parts (plan_prec).
   int64_t plan_units = 0, plan_cap = 0;
   bool fine = false, prec = false;
 };

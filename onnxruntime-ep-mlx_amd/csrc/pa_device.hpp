@@ -363,7 +363,8 @@ struct AttnParams {
   // partials instead, part 3 + slot of an item leaving its rows at slot * kPrefillRows; plan_cap
   // slots.  plan_split[i] is then 2 + n + 32 * (first slot) for an item of n parts.
   int32_t plan_units, plan_fine, plan_cap;
-  // P.V over images with the probabilities in two fp16 parts (about 22 bits)
+  // P.V over images with the probabilities in two parts (bf16: 16 bits at every size, against raw
+  // values; fp16: 22 bits from 2^-2 of the lazy maximum up, to within 2^-25 below)
   int32_t plan_prec;
   // GroupQueryAttention forms (VALU kernel; the others take none of them): key_limit[b] bounds
   // the keys of sequence b (its length, below past + query rows for a ragged first prompt); bias

@@ -629,7 +629,10 @@ __device__ __forceinline__ void img_issue(MxBufT<KB, D>& buf, int wave, int lane
 // F8S: fp8 pages (images of the dequantised rows in fp16, keys and values each under a per-step
 // power of two): the query rows go to fp16 under a per-row power of two as for INTC, and each
 // step's key exponent joins the softmax scale of the step.
-// PREC: P.V takes the probabilities as fp16 hi + lo parts (AttnParams::plan_prec).
+// PREC: P.V takes the probabilities in two parts (AttnParams::plan_prec), as the grid kernels of the
+// same calls do: fp16 hi + lo, or bf16 hi + lo against the bf16 values as they are (kRaw).  (Both parts
+// of an fp16 pair end at 2^-25, so below 2^-8 it holds fewer bits than a bf16 pair and below 2^-25
+// none, which values 2^26 times their neighbours would show.)
 // Workgroups per CU: two, bound by registers and from head 128 on by LDS; three to four at head 64
 // and up to three at 96 (33 and 49 KB of LDS).
 constexpr int mx_max_waves(bool img, int d) { return !img ? 2 : d == 64 ? 4 : d == 96 ? 3 : 2; }
@@ -642,7 +645,9 @@ prefill_mx_kernel(const AttnParams p) {
   using KT = typename std::conditional<INTC || F8S, TF16, TT>::type;  // score operand type
   // bf16 pages over images: steps may be wide (raw bf16 values, see kImgWideTag).  Head 256 keeps
   // one loop (its image kernel is at the register limit; a second loop instance spills).
-  constexpr bool kWide = IMG && !INTC && !F8S && std::is_same<TT, TBF16>::value && D <= 128;
+  constexpr bool kRaw = PREC && std::is_same<TT, TBF16>::value;
+  constexpr bool kWide =
+      IMG && !INTC && !F8S && std::is_same<TT, TBF16>::value && D <= 128 && !kRaw;
   constexpr int ROWS = kPrefillRows;
   static_assert(ROWS == 128, "four wavefronts of 32 rows");
   static_assert(IMG ? img_head(D) : D == 128, "images at heads 64 / 96 / 128 / 256, in-loop staging at 128");
@@ -881,7 +886,7 @@ prefill_mx_kernel(const AttnParams p) {
     int dsh = 0;
     bool pv_on = true;
     bool wide = false;
-    if constexpr (IMG) {
+    if constexpr (IMG && !kRaw) {
       if constexpr (kWideLoop) {  // raw bf16 values (see kImgWideTag); sj is the step's exponent
         wide = sj > kImgWideTag / 2;
         if (wide) sj -= kImgWideTag;
@@ -961,6 +966,35 @@ prefill_mx_kernel(const AttnParams p) {
         }
         return;
       }
+    }
+    if constexpr (kRaw) {
+      const float m0 = (m_run == kNegInf) ? 0.0f : m_run;
+      u32x4 ph[2 * KB], pl[2 * KB];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          float pv[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const float xv = x[kb][8 * half + i];
+            pv[i] = __builtin_amdgcn_exp2f(CAP ? xv - m0 : __builtin_fmaf(xv, sl2, -m0));
+            l_part += pv[i];
+          }
+          bf16x8 h8, l8;
+          TBF16::split8(pv, h8, l8);
+          ph[2 * kb + half] = __builtin_bit_cast(u32x4, h8);
+          pl[2 * kb + half] = __builtin_bit_cast(u32x4, l8);
+        }
+#pragma unroll
+      for (int t = 0; t < 2 * KB; ++t)
+#pragma unroll
+        for (int nt = 0; nt < NQ; ++nt) {
+          const u32x4 vv = buf.v[t][nt][lane];
+          o[nt] = mfma32<TBF16>(vv, ph[t], o[nt]);
+          o[nt] = mfma32<TBF16>(vv, pl[t], o[nt]);
+        }
+      return;
     }
     const float msafe = ((m_run == kNegInf) ? 0.0f : m_run) + (float)dsh;
     const _Float16 lw = (_Float16)(float)(1 << dsh);
@@ -1048,7 +1082,7 @@ prefill_mx_kernel(const AttnParams p) {
     else
       steps(std::false_type{});
 #pragma unroll
-    for (int nt = 0; nt < NQ; ++nt) sv[nt] = s_acc;
+    for (int nt = 0; nt < NQ; ++nt) sv[nt] = kRaw ? 0 : s_acc;
   } else {
     PageWindow pw;
     window_at(pw, w, min(div_bs(t_first, w), w.max_blocks - 1), lane);
@@ -1384,7 +1418,9 @@ __device__ __forceinline__ void img_store(const AttnParams& p, ImgGroup<NT, D>& 
   constexpr int KB = img_keys(D) / 32, CH = ImgGroup<NT, D>::CH, NQ = D / 32;
   constexpr int SB = img_step_bytes(D);
   // bf16 pages take a per-step scale; fp16 pages and integer codes (exact in fp16) go as they are
+  // (bf16 under plan_prec goes as it is too: the prefill kernel's kRaw products)
   constexpr bool BF = std::is_same<TT, TBF16>::value && KC == kImgT;
+  const bool scaled = BF && !p.plan_prec;
   const int tid = threadIdx.x, grp = tid / 256, r = g.r, q = g.q;
   char* dst = p.vimg + (g.hb * p.img_steps + g.j) * (int64_t)SB;
   auto store_keys = [&]() {
@@ -1402,7 +1438,7 @@ __device__ __forceinline__ void img_store(const AttnParams& p, ImgGroup<NT, D>& 
     e = wave_max_nonneg(f8_step_exp_biased(f8_chunks_absmax<CH>(g.vx) * fabsf(g.vs)));
     ek = wave_max_nonneg(f8_step_exp_biased(f8_chunks_absmax<CH>(g.kx) * fabsf(g.ks)));
   }
-  if constexpr (BF) {
+  if (scaled) {
     // largest magnitude and smallest nonzero magnitude (zeros read as 0x7fff), as bit patterns
     uint32_t mx = 0, mn = 0x7fff7fffu;
 #pragma unroll
@@ -1422,14 +1458,14 @@ __device__ __forceinline__ void img_store(const AttnParams& p, ImgGroup<NT, D>& 
   __syncthreads();
   if ((tid & 63) == 0) {
     atomicMax(&emax[grp], e);
-    if (KC == kImgF8 || BF) atomicMax(&emax[NT / 256 + grp], ek);
+    if (KC == kImgF8 || scaled) atomicMax(&emax[NT / 256 + grp], ek);
   }
   __syncthreads();
   // bf16: s = emax - 141 puts the largest value into [2^14, 2^15) of fp16; fp16: s = 0.  A wide
   // bf16 step (nonzero values kImgWideSpan or more binades apart) keeps its values as they are.
-  int sc = BF ? max(emax[grp] - 141, -112) : 0;
+  int sc = scaled ? max(emax[grp] - 141, -112) : 0;
   // (heads up to 128: the prefill kernel at head 256 has no loop for wide steps)
-  const bool wide = BF && D <= 128 && emax[grp] - (255 - emax[NT / 256 + grp]) >= kImgWideSpan;
+  const bool wide = scaled && D <= 128 && emax[grp] - (255 - emax[NT / 256 + grp]) >= kImgWideSpan;
   if constexpr (KC == kImgF8) {
     // fp8: code x page scale x 2^-s in fp16 (keys under their own s), both exponents to vstep
     const int sv = emax[grp] > 0 ? emax[grp] - 256 : 0;
@@ -1447,7 +1483,7 @@ __device__ __forceinline__ void img_store(const AttnParams& p, ImgGroup<NT, D>& 
     sc += kImgWideTag;
     if (g.step_live && (tid & 255) == 0) p.img_wide[g.hb] = p.img_epoch;
   }
-  if (BF && !wide) {
+  if (scaled && !wide) {
     // bf16 exponent E -> fp16 exponent E - 112 - s: subtract (112 + s) << 7 from the magnitude
     // bits (saturating: values below the fp16 range flush towards zero), shift into place
     const unsigned short bias = (unsigned short)((112 + sc) << 7);

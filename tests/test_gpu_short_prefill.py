@@ -55,3 +55,26 @@ def test_error_is_the_output_rounding(shape, dtype, most):
                         m.rows(v, "v", 0, past + n)).reshape(n, H * d)
     assert ((out[:n].double() - want).norm() / want.norm()).item() <= (
         most * 2 ** 0.5 if dtype == "float16" and d == 128 else most)
+
+
+@pytest.mark.parametrize("heads,kv,head", [(32, 8, 128), (64, 8, 64), (16, 4, 96)])
+def test_small_probabilities_of_large_values(heads, kv, head):
+    """bf16 keeps its values' whole exponent range, and their weights need theirs: 64 keys of weight 1
+    and values in [1, 2), then keys whose weights of 2^-26.5 meet values of 2^26 times as much.  The
+    output is rounded to bf16 (2^-9 of it); hi + lo probabilities add 2^-16."""
+    import torch
+    n = 900 if head == 96 else 500
+    m = Mixed(heads, kv, head, 16, [n], [0])
+    m.q.zero_()
+    m.q.view(n, heads, head)[..., 0] = 1.0
+    k, v = m.k.view(n, kv, head), m.v.view(n, kv, head)
+    k.zero_()
+    k[64:, :, 0] = -26.5 * np.log(2.0) * head ** 0.5
+    v.uniform_(1.0, 2.0, generator=torch.Generator(device="cuda").manual_seed(head))
+    v[64:] *= 2.0 ** 26
+    out = m.call()[0].double().view(n, kv, heads // kv, head)
+    s = torch.einsum("lkd,d->kl", k.double(), m.q.view(n, heads, head)[0, 0].double()) * head ** -0.5
+    w = s.exp()  # the same for every row: running sums give all of them
+    want = (w.T[..., None] * v.double()).cumsum(0) / w.cumsum(1).T[..., None]
+    err = ((out - want[:, :, None]).abs() / want[:, :, None]).amax().item()
+    assert err <= 2.0 ** -8, err
