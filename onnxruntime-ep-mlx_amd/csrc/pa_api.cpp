@@ -386,12 +386,14 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
     const int64_t live_keys =
         b->max_context_len > 0 ? std::min<int64_t>(b->max_context_len, ctx) : (int64_t)ctx;
     // a batch of fewer items than slots, over images of rows in T (bf16 images at head 256 hold one
-    // exponent per step, where the grid kernel takes the raw values: not there)
+    // exponent per step, where the grid kernel takes the raw values: not there), of a context that the
+    // caller bounds: the capacity says nothing of the keys there are, and images of all of it could
+    // cost any multiple of the grid launch
     const bool small = rich && PA_PREFILL_IMAGES && images && !bias && !intc && units < target &&
                        pa::img_head(c->head_dim) &&
                        !(act == PA_DTYPE_BFLOAT16 && c->head_dim > 128) &&
                        pa::prefill_mfma_supported(c->head_dim, act, c->dtype) &&
-                       short_planned(units, live_keys) &&
+                       b->max_context_len > 0 && short_planned(units, live_keys) &&
                        (int64_t)b->batch * c->kv_heads *
                                ((live_keys + pa::img_keys(c->head_dim) - 1) / pa::img_keys(c->head_dim)) *
                                pa::img_step_bytes(c->head_dim) <= kImgMaxBytes;

@@ -105,3 +105,20 @@ def test_context_bound_below_the_host_metadata_is_refused():
     node, io, keep = _paged([1000, 40], 64, 128, bound=-1)
     rc = lib.pa_paged_attention(C.byref(node), C.byref(io), C.c_void_p(0x2000), 1 << 40, None)
     assert rc == capi.PA_ERR_INVALID_ARGUMENT
+
+
+def test_short_prefills_plan_images_of_a_bounded_context_only():
+    """5 prompts of 100 tokens (160 row blocks, below the workgroup slots) over a 32,768-position table:
+    without a bound on their contexts the call keeps the grid launch and asks for no images (5 x 8 x 512
+    steps); with host metadata or a bound it may plan them."""
+    lib = capi.load()
+
+    def size(**kw):
+        node, io, keep = _paged([1900] * 5, 100, 2048, H=32, cache=capi.PA_DTYPE_BFLOAT16, **kw)
+        return lib.pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io))
+
+    images = 5 * 8 * 32 * STEP_BYTES
+    partials = 500 * 32 * 128 * 4 * 5  # fp32 rows of at most 5 chunks
+    assert size(host=False) < partials
+    assert images <= size(host=True) < images + (100 << 20)
+    assert size(host=False, bound=2000) == size(host=True)
