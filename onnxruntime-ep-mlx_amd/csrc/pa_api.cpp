@@ -282,18 +282,48 @@ bool latent_wide(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtyp
                                    pa::latent_wide_row_blocks(a->num_heads, mq));
 }
 
+// Context chunk of the grid-order prefill of `units` (row block, sequence, kv-head) items: as many
+// chunks as fill the workgroup slots.
+int64_t grid_chunk(int64_t units, int64_t slots, int ctx, int head_dim) {
+  const int64_t splits = (slots + units - 1) / units;
+  const int64_t ch = (ctx + splits - 1) / splits, step = pa::prefill_key_step(head_dim);
+  return std::min<int64_t>(std::max<int64_t>((ch + step - 1) / step * step, 256), INT32_MAX / 2);
+}
+
 // Whether a batch of fewer items than workgroup slots runs the planned image prefill all the same
-// (given the workspace).  The plan, images and merge launches cost about 12 us more than the grid
-// launch and its reduce, so a batch of few row blocks or short contexts stays there.  A call by
-// items x longest context, planned / grid: bf16 32 heads of 128: 56 x 1200 47.0 / 38.1 us, 128 x 512
-// 42.9 / 46.9, 224 x 200 37.6 / 28.4, 224 x 1200 64.3 / 74.8, 376 x 1500 69.3 / 90.4; fp16 28 heads
-// of 128: 44 x 1200 40.1 / 35.1, 112 x 2512 55.4 / 64.0, 448 x 4048 142 / 216; fp16 24 heads of 256:
-// 96 x 512 53.4 / 61.5, 384 x 4048 272 / 542; bf16 64 heads of 64: 128 x 1064 43.8 / 43.4, 256 x 512
-// 36.2 / 51.8.
+// (given the workspace): where the estimated time of its launches (images of every live key, the keys
+// that a slot walks when all share the work) is below the grid launch's (the keys of its chunks, cut
+// from the table's capacity, over its one or two workgroups a CU; the items' set-up; the partial rows
+// of every chunk).  seen: keys that a row block sees, fewer than the live ones under a window.
+// The figures (us, us a key and an item, head 256 apart) fit 6,880 calls timed both ways: fp16 and
+// bf16, 1 .. 40 row blocks a sequence, 96 .. 500 items, pasts of 0 .. 3000 keys, windows, tables of 1, 2
+// and 8 times the context.  The choice is 0.75 % off the better of the two on average, 15 % at worst
+// against the grid (always planned: 430 %).  Planned / grid: bf16 32 heads of 128, 60 x 29 tokens
+// after 1000 197 / 141, 38 x 29 after 3000 in a window of 128 233 / 64; 2 x 512 after 1000 73 / 84, 2000
+// tokens 94 / 126; fp16 24 heads of 256, 10 x 253 after 3000 390 / 742; bf16 64 heads of 64, 2 x 253
+// after 1000 50 / 68.
 #ifndef PA_R2_UNITS
 #define PA_R2_UNITS 96
 #endif
-bool short_planned(int64_t units, int64_t live) { return units >= PA_R2_UNITS && live >= 320; }
+bool short_planned(int64_t units, int64_t slots, int ctx, int64_t live, int64_t seen,
+                   int64_t image_rows, int head_dim) {
+  if (units < PA_R2_UNITS || live < 320) return false;
+  const bool big = head_dim > 128;
+  const double chunk = (double)grid_chunk(units, slots, ctx, head_dim);
+  const double chunks = std::ceil((double)live / chunk);
+  // workgroups with work a slot: between their mean and its round up
+  const double each = (double)units * std::max((double)seen / chunk, 1.0) / (double)(big ? slots / 2 : slots);
+  const double grid_keys =
+      std::min(chunk, (double)seen) * std::max(1.0, (each + std::ceil(each)) / 2);
+  const double plan_keys = std::max((double)units * (double)seen / (double)slots,
+                                    (double)std::min<int64_t>(seen, PA_FINE_MIN));
+  const double rows = chunks > 1.0 ? chunks : 0.0;  // partial rows of an item, in items
+  const double grid = (big ? 0.083 : 0.042) * grid_keys +
+                      (double)units * (big ? 0.08 + 0.055 * rows : 0.05 + 0.03 * rows);
+  const double plan = (big ? 0.11 : 0.042) * plan_keys + 1.8e-6 * (double)image_rows * head_dim +
+                      (head_dim == 128 ? 12.0 : 5.0);  // (beyond the grid launch's own start)
+  return plan < grid;
+}
 
 // rich: plans that need more workspace than the plain one of the same call are allowed; run_attention
 // takes them where the caller's workspace holds them (the size queries ask for that much) and the
@@ -389,11 +419,17 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
     // exponent per step, where the grid kernel takes the raw values: not there), of a context that the
     // caller bounds: the capacity says nothing of the keys there are, and images of all of it could
     // cost any multiple of the grid launch
+    const int64_t seen_keys =
+        a->local_window_size > 0
+            ? std::min<int64_t>(live_keys, (int64_t)a->local_window_size + pa::kPrefillRows / g)
+            : live_keys;
     const bool small = rich && PA_PREFILL_IMAGES && images && !bias && !intc && units < target &&
                        pa::img_head(c->head_dim) &&
                        !(act == PA_DTYPE_BFLOAT16 && c->head_dim > 128) &&
                        pa::prefill_mfma_supported(c->head_dim, act, c->dtype) &&
-                       b->max_context_len > 0 && short_planned(units, live_keys) &&
+                       b->max_context_len > 0 &&
+                       short_planned(units, target, ctx, live_keys, seen_keys,
+                                     (int64_t)b->batch * c->kv_heads * live_keys, c->head_dim) &&
                        (int64_t)b->batch * c->kv_heads *
                                ((live_keys + pa::img_keys(c->head_dim) - 1) / pa::img_keys(c->head_dim)) *
                                pa::img_step_bytes(c->head_dim) <= kImgMaxBytes;
@@ -442,11 +478,7 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
     } else if (units >= target) {
       chunk = (int)std::min<int64_t>(((int64_t)ctx + 31) / 32 * 32, INT32_MAX / 2);
     } else {
-      const int64_t splits = (target + units - 1) / units;
-      int64_t ch = (ctx + splits - 1) / splits;
-      const int64_t step = pa::prefill_key_step(c->head_dim);
-      chunk = (int)std::min<int64_t>(std::max<int64_t>((ch + step - 1) / step * step, 256),
-                                     INT32_MAX / 2);
+      chunk = (int)grid_chunk(units, target, ctx, c->head_dim);
     }
   }
   // Byte-coded pages that did not get the planned launch over images: the VALU kernel.

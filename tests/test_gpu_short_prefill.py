@@ -7,15 +7,16 @@ from test_gpu_mixed_batch import Mixed
 
 pytestmark = pytest.mark.gpu
 
-# heads, kv, head, block, new tokens, past: from the first batch the rule takes (96 items, 320 keys)
-# and just below it to whole rounds of slots, one long item among short ones (16 parts), empty
-# sequences, a single token and last row blocks of one row
+# heads, kv, head, block, new tokens, past: from the first batch the rule takes (96 items, 320 keys at
+# head 64) and just below it to whole rounds of slots, one long item among short ones (16 parts), empty
+# sequences, a single token and last row blocks of one row; at head 128 the grid launch keeps the first
 SHAPES = [
     (32, 8, 128, 16, [384], [0]), (32, 8, 128, 16, [353], [0]), (32, 8, 128, 16, [320], [0]),
     (28, 4, 128, 16, [512], [2000]), (28, 4, 128, 32, [1500, 0, 1, 33], [0, 5, 300, 7]),
     (8, 1, 128, 16, [1601, 17], [0, 30000]), (64, 8, 64, 16, [250, 250], [1000, 4000]),
     (64, 8, 64, 256, [511], [0]), (8, 4, 96, 16, [2000, 700], [100, 2500]),
     (24, 4, 256, 16, [513], [700]), (24, 4, 256, 32, [100, 90, 110, 200], [3000, 0, 500, 129]),
+    (32, 8, 128, 16, [500], [0]), (64, 8, 64, 16, [177], [143]), (64, 8, 64, 16, [176], [144]),
 ]
 FORMS = [dict(rot=32), dict(dtype="float16", rot=32),
          dict(dtype="float16", window=700, softcap=20.0, sink=True), dict(window=130, sink=True)]

@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes as C
 
 import numpy as np
+import pytest
 
 from onnxruntime_ep_mlx_amd import _capi as capi
 
@@ -50,7 +51,7 @@ def test_gqa_integer_present_images_follow_total_not_capacity():
 
 
 def _paged(past, nq, max_blocks, bs=16, KV=8, H=64, d=128, host=True, bound=0,
-           cache=capi.PA_DTYPE_FP8_E4M3):
+           cache=capi.PA_DTYPE_FP8_E4M3, act=capi.PA_DTYPE_BFLOAT16, window=-1):
     B = len(past)
     cum = np.concatenate([[0], np.cumsum([nq] * B)]).astype(np.int32)
     past = np.asarray(past, np.int32)
@@ -59,12 +60,12 @@ def _paged(past, nq, max_blocks, bs=16, KV=8, H=64, d=128, host=True, bound=0,
     keep = [cum, past, bt]
     c = capi.PaCache(FAKE, FAKE, FAKE, FAKE, nb, bs, KV, d, cache)
     T = int(cum[-1])
-    io = capi.PaIO(capi.PA_DTYPE_BFLOAT16, T, H * d, FAKE, FAKE, FAKE, c, FAKE, FAKE, FAKE,
+    io = capi.PaIO(act, T, H * d, FAKE, FAKE, FAKE, c, FAKE, FAKE, FAKE,
                    B, max_blocks, None, None, 0, 0, None, None, None, None,
                    cum.ctypes.data if host else None, past.ctypes.data if host else None,
                    bt.ctypes.data if host else None, None, FAKE, None, None,
                    nq if not host else 0, bound)
-    node = capi.PaNode(H, KV, 0.0, 0.0, -1, 0, 0, 0, 1, 1e-6)
+    node = capi.PaNode(H, KV, 0.0, 0.0, window, 0, 0, 0, 1, 1e-6)
     return node, io, keep
 
 
@@ -122,3 +123,28 @@ def test_short_prefills_plan_images_of_a_bounded_context_only():
     assert size(host=False) < partials
     assert images <= size(host=True) < images + (100 << 20)
     assert size(host=False, bound=2000) == size(host=True)
+
+
+# heads, kv-heads, head, sequences, new tokens, past, window, table positions (0: what is needed); both
+# launches timed on an MI355X, us, planned / grid
+@pytest.mark.parametrize("H,KV,d,B,nq,past,window,table,planned", [
+    (32, 8, 128, 60, 29, 1000, -1, 0, False),   # 197 / 141: images read by one row block each
+    (32, 8, 128, 38, 29, 3000, 128, 0, False),  # 233 / 64: of keys that no row sees
+    (32, 8, 128, 15, 125, 3000, 128, 0, False),  # 129 / 87
+    (64, 8, 64, 38, 13, 3000, 128, 0, False),   # 125 / 53
+    (32, 8, 128, 4, 125, 3000, -1, 0, False),   # 87 / 75
+    (32, 8, 128, 2, 512, 1000, -1, 0, True),    # 73 / 84
+    (32, 8, 128, 1, 2000, 4000, 128, 0, True),  # 52 / 86: a window over many row blocks
+    (64, 8, 64, 8, 45, 1000, -1, 0, True),      # 45 / 65
+    (32, 8, 128, 4, 125, 1000, -1, 8960, True),  # 55 / 69: chunks cut from a table of 8 contexts
+])
+def test_short_prefills_weigh_images_against_what_reads_them(H, KV, d, B, nq, past, window, table,
+                                                             planned):
+    lib = capi.load()
+    for act in (capi.PA_DTYPE_BFLOAT16, capi.PA_DTYPE_FLOAT16):
+        n = []
+        for host in (True, False):  # without a bound: the grid launch
+            node, io, keep = _paged([past] * B, nq, max(-(-(past + nq) // 16), table // 16), KV=KV,
+                                    H=H, d=d, host=host, cache=act, act=act, window=window)
+            n.append(lib.pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io)))
+        assert (n[0] != n[1]) == planned
