@@ -335,6 +335,7 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
                int chunk, bool linear = false, int linear_cap = 0, bool images = true,
                bool bias = false, const HostLens& hl = HostLens(), bool rich = false) {
   Plan pl{};
+  const bool automatic = kind == 0;
   // The LATENT layout (values = leading dims of the key rows): its matrix-core kernel (kind 5)
   // where it covers the head sizes and dtypes, else the VALU kernel.
   if (c->value_cache == nullptr || (a->v_head_size > 0 && a->v_head_size != c->head_dim)) {
@@ -423,7 +424,7 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
         a->local_window_size > 0
             ? std::min<int64_t>(live_keys, (int64_t)a->local_window_size + pa::kPrefillRows / g)
             : live_keys;
-    const bool small = rich && PA_PREFILL_IMAGES && images && !bias && !intc && units < target &&
+    const bool small = rich && automatic && PA_PREFILL_IMAGES && images && !bias && !intc && units < target &&
                        pa::img_head(c->head_dim) &&
                        !(act == PA_DTYPE_BFLOAT16 && c->head_dim > 128) &&
                        pa::prefill_mfma_supported(c->head_dim, act, c->dtype) &&

@@ -148,3 +148,20 @@ def test_short_prefills_weigh_images_against_what_reads_them(H, KV, d, B, nq, pa
                                     H=H, d=d, host=host, cache=act, act=act, window=window)
             n.append(lib.pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io)))
         assert (n[0] != n[1]) == planned
+
+
+def test_forced_prefill_kind_splits_short_batches_over_the_grid():
+    """pa_attention_ex with kind 2: the planned launch once the batch fills the GPU, else context chunks;
+    the automatic choice may plan a short batch over images."""
+    lib = capi.load()
+    B, nq, past, KV, H, d, bs = 2, 512, 1000, 8, 32, 128, 16
+    mb = -(-(past + nq) // bs)
+    cache = capi.PaCache(FAKE, FAKE, None, None, B * mb, bs, KV, d, capi.PA_DTYPE_BFLOAT16)
+    batch = capi.PaBatch(FAKE, FAKE, FAKE, None, B, mb, B * nq, nq, 0, past + nq)
+    attn = capi.PaAttn(H, 0.0, 0.0, -1, 1, None)
+    size = lambda kind: lib.pa_attention_workspace_bytes_ex(
+        C.byref(cache), C.byref(batch), C.byref(attn), capi.PA_DTYPE_BFLOAT16, kind, 0)
+    chunks = 2  # 256 row blocks, 512 workgroup slots
+    partials = B * nq * H * chunks * (d * 4 + 8)
+    assert partials <= size(2) < partials + 1024
+    assert size(0) > B * KV * 24 * STEP_BYTES
