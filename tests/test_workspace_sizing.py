@@ -165,3 +165,42 @@ def test_forced_prefill_kind_splits_short_batches_over_the_grid():
     partials = B * nq * H * chunks * (d * 4 + 8)
     assert partials <= size(2) < partials + 1024
     assert size(0) > B * KV * 24 * STEP_BYTES
+
+
+def _latent(past, H, table=0, bs=16, nq=1, host=True):
+    B = len(past)
+    cum = (np.arange(B + 1) * nq).astype(np.int32)
+    past = np.asarray(past, np.int32)
+    mb = -(-max(int(past.max()) + nq, table) // bs)
+    cache = capi.PaCache(FAKE, None, None, None, B * mb, bs, 1, 576, capi.PA_DTYPE_BFLOAT16)
+    io = capi.PaIO(capi.PA_DTYPE_BFLOAT16, B * nq, H * 576, FAKE, FAKE, None, cache, FAKE, FAKE, FAKE, B,
+                   mb, None, None, 0, 0, None, None, None, None, cum.ctypes.data if host else None,
+                   past.ctypes.data if host else None, FAKE if host else None, None, FAKE, None, None,
+                   0 if host else nq, 0)
+    node = capi.PaNode(H, 1, 192.0**-0.5, 0.0, -1, 0, 0, 0, 1, 1e-6, 512, 1)
+    return capi.load().pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io))
+
+
+SEGMENTS = 2 * 256 * 64 * (512 * 4 + 8) + 256 * 16  # partials and list of the 64-row blocks
+
+
+# heads, sequences, keys; 64-row blocks / smaller ones, us on an MI355X
+@pytest.mark.parametrize("H,B,keys,wide", [
+    (16, 4, 64, False),    # 18.3 / 16.2
+    (16, 64, 96, False),   # 23.4 / 19.0
+    (16, 64, 128, False),  # 23.5 / 20.9
+    (16, 4, 128, True),    # 18.9 / 19.5
+    (16, 64, 256, True),   # 27.3 / 28.6
+    (32, 64, 96, True),    # 29.7 / 30.0
+    (128, 16, 96, False),  # 33.5 / 29.7
+    (64, 32, 128, False),  # 33.2 / 31.8
+    (128, 8, 96, True),    # 26.9 / 27.8
+    (128, 48, 192, False),  # 51.3 / 40.8
+    (128, 32, 192, True),  # 37.5 / 38.5
+    (128, 64, 384, False),  # 59.7 / 55.4
+    (128, 64, 448, True),
+    (128, 66, 256, True),  # more than one round of the smaller blocks
+])
+def test_latent_blocks_follow_rows_and_keys(H, B, keys, wide):
+    n = _latent([keys - 1] * B, H)
+    assert (n == SEGMENTS) == wide, n
