@@ -295,9 +295,13 @@ bool latent_short(const pa_cache* c, const pa_batch* b, const pa_attn* a, int mq
   return 8 * rows >= eighths * full;
 }
 
-bool latent_wide(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act) {
+// (The 64-row blocks read every row from the pages, which only the caller's word or the operator's
+// host metadata can promise.)
+bool latent_wide(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act,
+                 const HostLens& hl) {
   const int mq = b->max_query_len > 0 ? b->max_query_len : std::max(b->num_tokens, 1);
-  return (int64_t)a->num_heads * mq >= PA_LATENT_WIDE_ROWS &&
+  const bool pages = ((b->flags & PA_BATCH_NEW_ROWS_IN_CACHE) || hl.cum) && !b->slot_mapping;
+  return pages && (int64_t)a->num_heads * mq >= PA_LATENT_WIDE_ROWS &&
          pa::latent_wide_supported(c->head_dim, a->v_head_size, act, c->dtype, c->block_size,
                                    b->max_blocks, b->batch,
                                    pa::latent_wide_row_blocks(a->num_heads, mq)) &&
@@ -369,7 +373,7 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
   }
   const int g = a->num_heads / c->kv_heads;
   const int mq = b->max_query_len > 0 ? b->max_query_len : std::max(b->num_tokens, 1);
-  if (kind == 5 && rich && chunk <= 0 && latent_wide(c, b, a, act)) {
+  if (kind == 5 && rich && chunk <= 0 && latent_wide(c, b, a, act, hl)) {
     pl.kind = 6;
     pl.chunk = 32;
     pl.max_splits = device_cus();
@@ -669,8 +673,9 @@ SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_
 
 // Whether a call whose plain plan is pl has no richer one (and the search for pl's chunk need not run
 // again to find that out).
-bool plain_only(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act, const Plan& pl) {
-  return pl.kind != 2 && !(pl.kind == 5 && latent_wide(c, b, a, act));
+bool plain_only(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act, const Plan& pl,
+                const HostLens& hl) {
+  return pl.kind != 2 && !(pl.kind == 5 && latent_wide(c, b, a, act, hl));
 }
 
 // Workspace of a call: what it needs to run, and with the plans that more workspace allows.
@@ -683,7 +688,7 @@ WsNeed ws_need(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
   WsNeed n;
   const Plan plain = make_plan(c, b, a, act, kind, chunk, linear, linear_cap, images, bias, hl);
   n.best = n.least = workspace_for(c, b, a, plain);
-  if (plain_only(c, b, a, act, plain)) return n;
+  if (plain_only(c, b, a, act, plain, hl)) return n;
   n.best = std::max(n.least, workspace_for(c, b, a, make_plan(c, b, a, act, kind, chunk, linear,
                                                                linear_cap, images, bias, hl, true)));
   return n;
@@ -854,7 +859,7 @@ int run_attention(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dty
   if (need > 0 && (!ws || ws_bytes < need))
     return fail(PA_ERR_INVALID_ARGUMENT, "workspace too small: need %zu bytes, got %zu", need,
                 ws_bytes);
-  if (!plain_only(c, b, a, act, pl)) {
+  if (!plain_only(c, b, a, act, pl, opts.host)) {
     const Plan pr = make_plan(c, b, a, act, kind, chunk, opts.linear_cap > 0, opts.linear_cap,
                               plan_images(opts), opts.bias != nullptr, opts.host, true);
     // (the wide LATENT kernel reads every row from the pages)

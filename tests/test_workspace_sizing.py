@@ -204,3 +204,19 @@ SEGMENTS = 2 * 256 * 64 * (512 * 4 + 8) + 256 * 16  # partials and list of the 6
 def test_latent_blocks_follow_rows_and_keys(H, B, keys, wide):
     n = _latent([keys - 1] * B, H)
     assert (n == SEGMENTS) == wide, n
+
+
+def test_latent_segments_are_asked_for_only_where_they_can_run():
+    """The 64-row blocks read every row from the pages: without host metadata (operator) or
+    PA_BATCH_NEW_ROWS_IN_CACHE (kernel entry), or with a slot mapping, they cannot run."""
+    lib = capi.load()
+    assert _latent([1000] * 4, 16) == SEGMENTS
+    assert _latent([1000] * 4, 16, host=False) < SEGMENTS // 8
+    cache = capi.PaCache(FAKE, None, None, None, 256, 16, 1, 576, capi.PA_DTYPE_BFLOAT16)
+    attn = capi.PaAttn(16, 0.1, 0.0, -1, 1, None, 512)
+    for flags, slots, wide in ((0, None, False), (capi.PA_BATCH_NEW_ROWS_IN_CACHE, None, True),
+                               (capi.PA_BATCH_NEW_ROWS_IN_CACHE, FAKE, False)):
+        batch = capi.PaBatch(FAKE, FAKE, FAKE, slots, 4, 64, 4, 1, flags, 0)
+        n = lib.pa_attention_workspace_bytes_ex(C.byref(cache), C.byref(batch), C.byref(attn),
+                                                capi.PA_DTYPE_BFLOAT16, 0, 0)
+        assert (n == SEGMENTS) == wide, (flags, n)
