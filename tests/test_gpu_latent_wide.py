@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 TOL = {BF16: 2.0**-7 / 12**0.5, F16: 2.0**-10 / 12**0.5}
 
 
-def check(H, new, past, bs=16, dtype=BF16, **kw):
+def check(H, new, past, bs=16, dtype=BF16, static=False, **kw):
     B = len(new)
     mb = -(-max(p + n for p, n in zip(past, new)) // bs) + 1
     c = make_latent_case(H, 576, 512, B * mb, bs, B, dtype=dtype, seed=H + B + sum(past) % 1000,
@@ -27,7 +27,7 @@ def check(H, new, past, bs=16, dtype=BF16, **kw):
                          **kw)
     print(f"latent wide H={H} new={new[:6]} past={past[:6]} bs={bs} dtype={dtype}", flush=True)
     ref, _, kc_ref, _ = orc.paged_attention_op(c)
-    out, kc, _ = run_gpu_op(c)
+    out, kc, _ = run_gpu_op(c, static_scratch=static)
     np.testing.assert_array_equal(kc, kc_ref)
     want = orc.decode(orc.encode(ref.astype(np.float32), dtype), dtype).astype(np.float64)
     err = orc.rel_l2(orc.decode(out, dtype).astype(np.float64), want)
@@ -61,3 +61,18 @@ def test_segments(H, past):
 def test_masks(window, softcap, sink, scale):
     check(48, [1, 9, 2], [600, 250, 0], window=window, softcap=softcap, scale=scale,
           head_sink=np.linspace(-1, 1, 48) if sink else None)
+
+
+# The library's 64 MiB hold no segments of 64-row blocks: 16- and 32-row blocks (pa_latent.hip) on the
+# same rows, in one chunk and in several
+@pytest.mark.parametrize("dtype", [BF16, F16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("H,new,past", [(16, [1, 1], [130, 2500]), (33, [1], [197]), (64, [1] * 3, [640] * 3),
+                                        (128, [1, 2], [131, 1900]), (16, [5, 70], [60, 300])])
+def test_smaller_blocks_in_the_static_workspace(H, new, past, dtype):
+    check(H, new, past, dtype=dtype, static=True)
+
+
+# contexts that keep the smaller blocks with any workspace
+@pytest.mark.parametrize("H,past", [(16, [0, 31, 63, 95]), (16, [127] * 16), (64, [100 + i % 28 for i in range(32)])])
+def test_short_contexts(H, past):
+    check(H, [1] * len(past), past)

@@ -35,6 +35,15 @@ def test_short_prefill(shape, form):
     m.check(*bounded)
 
 
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("shape", SHAPES)
+def test_grid_launch_of_the_same_batches(shape, form):
+    """Without a bound on their contexts they run on the grid launch."""
+    m = Mixed(*shape, **form)
+    m.check(*m.call(validate=False, max_query_len=max(m.new)))
+
+
 @pytest.mark.parametrize("dtype,most", [("bfloat16", 2.3e-3), ("float16", 2.9e-4)])
 @pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[3], SHAPES[6], SHAPES[9]])
 def test_error_is_the_output_rounding(shape, dtype, most):
