@@ -83,12 +83,15 @@ constexpr bool kIntCache<I8Cache> = true;
 template <>
 constexpr bool kIntCache<I4Cache> = true;
 
-// Elements per lane: NE = 4 covers head_dim <= 256, NE = 10 head_dim <= 640 (latent heads).
+// Elements per lane: NE = 1, 2, 4 cover head_dim <= 64, 128, 256, NE = 10 head_dim <= 640 (latent
+// heads).  (Bound by instruction issue: with the four of head 256 at every size one fp32 token of head
+// 64 took 13.1 us a call instead of 11.5, 64 of head 64 over 500 .. 1000 keys 136 instead of 116, four
+// 200-token fp16 prompts of head 80 155 instead of 126.)
 // NW wavefronts take keys w, w + NW, ... of the chunk, kGenKeys of them per round: their rows are
 // loaded together and their cross-lane sums interleave.  A round is a chain of two or three memory
 // latencies (block table, rows) and the sums, so a call of few (token, head) pairs takes as long as
 // its rounds: one fp32 token of 8 heads over 129 keys 79 us with one wavefront and one key at a
-// time, 10.8 with 16 (launch_generic_ne has the rule).
+// time, 8.9 with 16 (launch_generic_ne has the rule).
 template <int NE>
 constexpr int kGenKeys = NE <= 4 ? 8 : 2;
 template <typename TT, typename CT, int NE, int NW>
@@ -145,11 +148,14 @@ __global__ __launch_bounds__(64 * NW) void attn_generic_kernel(const AttnParams 
   const float cap = p.softcap;
   for (int64_t p0 = lo + wave; p0 < hi; p0 += NW * U) {
     float x[U], vv[U][NE];
+    const int left = (int)min(hi - p0, (int64_t)(NW * U));  // keys of the round from this one on
     {
       float part[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int64_t pos = min(p0 + NW * u, hi - 1);  // surplus keys weigh nothing below
+        // a surplus key repeats the last one: weight 0 below, and no values (theirs may be infinite)
+        const int64_t pos = min(p0 + NW * u, hi - 1);
+        const int vd = NW * u < left ? VD : 0;
         const void *kb, *vb;
         int64_t off;
         float ks = 1.0f, vs = 1.0f;
@@ -188,7 +194,7 @@ __global__ __launch_bounds__(64 * NW) void attn_generic_kernel(const AttnParams 
                                  : TT::to_f32(reinterpret_cast<const typename TT::raw*>(kb)[off + e]);
             part[u] += qv[k] * kv;
           }
-          if (e < VD)
+          if (e < vd)
             vv[u][k] = from_cache
                            ? CacheRead<CT>::at(vb, off, e, kIntCache<CT> ? vsv[k] : vs)
                            : TT::to_f32(reinterpret_cast<const typename TT::raw*>(vb)[off + e]);
@@ -222,11 +228,8 @@ __global__ __launch_bounds__(64 * NW) void attn_generic_kernel(const AttnParams 
     for (int u = 0; u < U; ++u) {
       const float w = exp2f(x[u] - msafe);
       l += w;
-      // a surplus key repeats the row's last one: weight 0, and its values, which may be infinite, left
-      // out (the test is the same for the whole wavefront)
-      if (u == 0 || p0 + NW * u < hi)
 #pragma unroll
-        for (int k = 0; k < NE; ++k) o[k] += w * vv[u][k];
+      for (int k = 0; k < NE; ++k) o[k] += w * vv[u][k];
     }
     m = mn;
   }
@@ -369,7 +372,7 @@ __global__ __launch_bounds__(NT) void split_reduce_kernel(const AttnParams p) {
   }
 }
 
-// Lanes hold head_dim / 64 elements: 4 up to 256, 10 up to 640.
+// Lanes hold head_dim / 64 elements: 1, 2 and 4 up to 64, 128 and 256, 10 up to 640.
 constexpr int kMaxHeadDim = 640;
 template <int NE>
 constexpr bool ne_covers(int d) { return d <= 64 * NE; }
@@ -416,6 +419,8 @@ hipError_t launch_generic_ne(const AttnParams& p, pa_dtype cache_dtype, hipStrea
 
 template <typename TT>
 hipError_t launch_generic_t(const AttnParams& p, pa_dtype cache_dtype, hipStream_t s) {
+  if (ne_covers<1>(p.head_dim)) return launch_generic_ne<TT, 1>(p, cache_dtype, s);
+  if (ne_covers<2>(p.head_dim)) return launch_generic_ne<TT, 2>(p, cache_dtype, s);
   return ne_covers<4>(p.head_dim) ? launch_generic_ne<TT, 4>(p, cache_dtype, s)
                                   : launch_generic_ne<TT, 10>(p, cache_dtype, s);
 }

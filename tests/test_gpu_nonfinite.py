@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 # key counts that leave a wavefront's last round short, full and with one key over: rounds hold 8
 # keys (2 beyond head 256) of each of 1, 4 or 16 wavefronts
-@pytest.mark.parametrize("dtype,head", [(orc.F32, 64), (orc.F16, 40), (orc.F32, 320)])
+@pytest.mark.parametrize("dtype,head", [(orc.F32, 64), (orc.F16, 40), (orc.F32, 96), (orc.F32, 200),
+                                        (orc.F32, 320)])
 @pytest.mark.parametrize("past", [[0, 1, 6, 7, 8, 14], [31, 62, 63, 64, 126, 127, 128, 300],
                                   list(range(0, 560, 7))])
 def test_infinite_last_value_on_the_valu_kernel(dtype, head, past):
