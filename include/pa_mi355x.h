@@ -199,8 +199,9 @@ size_t pa_attention_workspace_bytes_ex(const pa_cache* cache, const pa_batch* ba
  *   - other batches over pages in T: the LDS-shared prefill kernel (128 grouped query rows per
  *     workgroup; the planned launch -- longest-first units, long items split in two -- once the
  *     batch fills two workgroups per compute unit, over operand images when each (sequence,
- *     kv-head) has at least 4 row blocks; also from 96 such row blocks and 320 live keys on with the
- *     queried workspace, except bf16 at head 256);
+ *     kv-head) has at least 4 row blocks; with the queried workspace and a bound on the contexts
+ *     (max_context_len, or the operator's host metadata) also batches from 96 such row blocks and 320
+ *     live keys on, except bf16 at head 256, whose images are estimated to cost less than they save);
  *   - other batches over fp8 / int8 / int4 pages: the planned prefill over operand images (fp16
  *     rows of the live context, within 2 GiB of workspace; larger batches run it on groups of
  *     sequences whose images fit, one launch per group);
@@ -208,7 +209,8 @@ size_t pa_attention_workspace_bytes_ex(const pa_cache* cache, const pa_batch* ba
  *     the activation dtype, key rows of a multiple of 32 dims up to 640 and values of 128, 256
  *     or 512 dims (MLA 576 / 512): its matrix-core kernels, all heads served by one read of each
  *     row per 16 or 32 grouped query rows, and per 64 at 576 / 512 with 16 or more of them, the new
- *     rows in the pages, whole 16-row tiles per page and the queried workspace;
+ *     rows in the pages, whole 16-row tiles per page and the queried workspace, but for short contexts
+ *     that the smaller blocks take in one round;
  *   - fp32 activations, other head sizes, other LATENT shapes and forced split-K chunks over
  *     byte-coded pages: the VALU kernel.
  * batch->max_query_len = 0 is read as num_tokens. */
@@ -318,9 +320,10 @@ int pa_paged_attention(const pa_paged_attention_node* node, const pa_paged_atten
  * for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  Same contract as pa_paged_attention, except that the
  * workspace is a scratch buffer of PA_STATIC_SCRATCH_BYTES inside the library's code object on
- * each GPU (a file-scope __device__ array, resident until the process ends): a call whose
- * workspace (pa_paged_attention_workspace_bytes) exceeds it returns PA_ERR_UNSUPPORTED before
- * any device work.  No hipMalloc / hipFree or other allocating routine is called.  Every call
+ * each GPU (a file-scope __device__ array, resident until the process ends).  A call whose queried
+ * workspace (pa_paged_attention_workspace_bytes) exceeds it runs on a plainer plan that fits; one
+ * whose plainest plan does not fit returns PA_ERR_UNSUPPORTED before any device work.  (The partials
+ * of the 64-row MLA blocks alone fill it: captured MLA steps run in the smaller ones.)  No hipMalloc / hipFree or other allocating routine is called.  Every call
  * on one GPU shares that GPU's scratch: calls that overlap on one GPU (different streams, or
  * host threads) race and must be serialised by the caller; calls in stream order do not.  The
  * kernels need no cleared scratch (everything they read is written earlier in the same call). */

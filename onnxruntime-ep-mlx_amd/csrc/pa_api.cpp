@@ -566,7 +566,8 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
 }
 
 // Bytes of the partial rows: fp32 elements, except the planned prefill's halves, which are
-// stored as fp16 rows scaled by a power of two (store_rows with half_part).
+// stored as fp16 rows scaled by a power of two (store_rows with half_part).  A short planned prefill
+// (fine) leaves either, as its keys turn out: room for the larger.
 size_t part_o_bytes(const pa_cache* c, const Plan& pl) {
   if (pl.fine)
     return align256(std::max((size_t)pl.plan_items * 2 * pa::kPrefillRows * 2,
@@ -576,8 +577,9 @@ size_t part_o_bytes(const pa_cache* c, const Plan& pl) {
 }
 
 // Workspace: [partial O | partial (m, l)].
-// Planned prefill adds [unit list (2 per item, 4 int32 each) | unit count | split flag per item].
-// Operand images add [images | step value exponents].
+// Planned prefill adds [unit list (plan_units of 4 int32) | unit count | split flag per item].
+// Operand images add [images | step value exponents | wide flags]; the 64-row MLA blocks the list of
+// their merge (4 int32 per segment).
 size_t plan_bytes(const Plan& pl) {
   return align256((size_t)pl.plan_units * 4 * sizeof(int32_t)) + 256 +
          align256((size_t)pl.plan_items * sizeof(int32_t));

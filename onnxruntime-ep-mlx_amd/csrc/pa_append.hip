@@ -1051,7 +1051,8 @@ static void launch_rows(const AppendParams& p, hipStream_t s) {
   const int64_t chunks =
       ((int64_t)(do_q ? p.num_heads : 0) + kv + (p.value ? kv : 0)) * (p.head_dim / 8);
   const int64_t per = std::max<int64_t>((chunks + 63) / 64, 1);  // 64-lane passes per token
-  // As many passes per wavefront as leave kRowsWaves wavefronts (8 per SIMD is what fits).
+  // As many passes per wavefront as still leave about kRowsWaves wavefronts, four per SIMD; every token
+  // takes one at least (3079 tokens of 10 passes: two of 5 each).
   const int64_t want = (kRowsWaves + p.num_tokens - 1) / p.num_tokens;
   const int passes = (int)std::max<int64_t>(per / std::max<int64_t>(want, 1), 1);
   const int slices = (int)((per + passes - 1) / passes);

@@ -91,7 +91,7 @@ constexpr bool kIntCache<I4Cache> = true;
 // loaded together and their cross-lane sums interleave.  A round is a chain of two or three memory
 // latencies (block table, rows) and the sums, so a call of few (token, head) pairs takes as long as
 // its rounds: one fp32 token of 8 heads over 129 keys 79 us with one wavefront and one key at a
-// time, 8.9 with 16 (launch_generic_ne has the rule).
+// time, 8.7 with 16 (launch_generic_ne has the rule).
 template <int NE>
 constexpr int kGenKeys = NE <= 4 ? 8 : 2;
 template <typename TT, typename CT, int NE, int NW>
@@ -400,10 +400,10 @@ hipError_t launch_generic_nw(const AttnParams& p, pa_dtype cache_dtype, hipStrea
 
 // Wavefronts per (chunk, head, token): 16 while those workgroups fit the chip at once (512: two per
 // CU), then 4; beside at most 32 keys a workgroup holds one or two rounds at most and its meeting in
-// LDS costs more, so 4 and 1 there.  fp32, 8 heads of 64, a call with 16 / 4 / 1: one token over 2048
-// keys 21.2 / 36.4 / 109.8 us, 8 tokens over 600 22.3 / 37.0 / 110.7; 128 tokens over 128 keys 44.1 /
-// 33.2 / 83.7, 8 x 100 over 2048 1879 / 1567 / 2311; 16-token prompts 18.7 / 14.4 / 20.7 (one) and
-// 97.9 / 33.6 / 24.3 (32 of them).
+// LDS costs more, so 4 and 1 there.  fp32, 8 heads of 64, a paged call with 16 / 4 / 1: one token over
+// 2048 keys 25.1 / 42.0 / 132.6 us, 8 tokens over 600 25.9 / 42.6 / 133.2; 128 tokens over 128 keys 48.2 /
+// 39.6 / 94.2, 8 x 100 over 2048 2685 / 2000 / 2661; 16-token prompts 12.0 / 9.5 / 12.1 (one) and 89.9 /
+// 26.0 / 17.0 (32 of them).
 template <typename TT, int NE>
 hipError_t launch_generic_ne(const AttnParams& p, pa_dtype cache_dtype, hipStream_t s) {
   const int64_t groups = (int64_t)p.max_splits * p.num_heads * p.num_tokens;

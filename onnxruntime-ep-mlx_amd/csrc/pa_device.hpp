@@ -359,7 +359,7 @@ struct AttnParams {
   // item key ranges start and split at multiples of it.
   int32_t plan_items, plan_rbs, plan_slots, plan_step;
   // Capacity of the unit list.  plan_fine (image launches): short batches -- fewer than
-  // kPlanSplitMin keys per workgroup slot -- split their items into up to kFineParts parts with fp32
+  // PA_PLAN_SPLIT_MIN keys per workgroup slot -- split their items into up to kFineParts parts with fp32
   // partials instead, part 3 + slot of an item leaving its rows at slot * kPrefillRows; plan_cap
   // slots.  plan_split[i] is then 2 + n + 32 * (first slot) for an item of n parts.
   int32_t plan_units, plan_fine, plan_cap;
@@ -539,7 +539,7 @@ bool latent_mfma_supported(int head_dim, int v_head_dim, pa_dtype act, pa_dtype 
 // 16-row groups per LATENT workgroup for H heads and max_query_len mq.
 inline int latent_row_groups(int heads, int mq) { return (int64_t)heads * mq >= 32 ? 2 : 1; }
 hipError_t launch_latent(const AttnParams& p, pa_dtype act, pa_dtype cache_dtype, hipStream_t s);
-// MLA rows against blocks of 64 grouped query rows (pa_latent.hip); max_splits: its workgroups, each
+// MLA rows against blocks of 64 grouped query rows (pa_latent_wide.hip); max_splits: its workgroups, each
 // with two partial slots of kLatWideRows rows of kLatWideDims.
 constexpr int kLatWideRows = 64, kLatWideDims = 512;
 bool latent_wide_supported(int head_dim, int v_head_dim, pa_dtype act, pa_dtype cache_dtype,

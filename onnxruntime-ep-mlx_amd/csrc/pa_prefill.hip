@@ -620,9 +620,6 @@ __device__ __forceinline__ void img_issue(MxBufT<KB, D>& buf, int wave, int lane
 
 // IMG: value operands from the per-(sequence, kv-head) value images (AttnParams::vimg), staged
 // by direct LDS loads one step ahead; otherwise loaded, converted and regrouped in the loop.
-#ifndef PA_IMG_WAVES
-#define PA_IMG_WAVES 2
-#endif
 // INTC: integer pages (images of fp16 codes): per-channel / per-tensor key scales fold into the
 // query, normalised per row by a power of two whose exponent joins the row's softmax scale; the
 // scores run on fp16 products; value scales multiply the output per dim before normalisation.
@@ -1930,7 +1927,7 @@ hipError_t launch_prefill_merge(const AttnParams& p, hipStream_t s) {
 
 }  // namespace
 
-// Planned prefill: plan (one workgroup), the prefill kernel over 2 * plan_items unit slots
+// Planned prefill: plan (one workgroup), the prefill kernel over plan_units unit slots
 // (workgroups past the planned count exit at once), then the merge of the split items.
 hipError_t launch_prefill_planned(const AttnParams& p, pa_dtype act, pa_dtype cache_dtype,
                                   hipStream_t s) {
