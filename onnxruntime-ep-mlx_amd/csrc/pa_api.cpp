@@ -275,8 +275,10 @@ int latent_chunk(const pa_cache* c, const pa_batch* b, const pa_attn* a, const H
 // sequences 37.0 / 55.7 against 45.0 / 93.2, 64 58.0 / - / 147 against 51.4 / - / 371; prompts, 128 heads
 // of 100 tokens after 1000 93 against 201, two of 256 after 2000 526 against 1404.
 //
-// Not where the contexts are so short that the smaller blocks take each in one chunk and all of them
-// fit the chip at once, without partials and their merge, which the segments still cut: 16-row blocks
+// Not where the contexts, and the tables behind them, are so short that the smaller blocks take each in
+// one chunk and all of them fit the chip at once, without partials and their merge, which the segments
+// still cut (behind a table of 8192 keys 128 heads, 64 sequences of 96 keys take 60.5 us in the smaller
+// blocks, whose grid covers the table, against 45.9): 16-row blocks
 // up to 96 keys (16 heads, 64 sequences of 64 keys 19.6 against 17.0 us, of 96 23.4 / 19.0) and from 16
 // sequences up to 128 (23.5 / 20.9; 8 sequences 19.5 / 20.0); 32-row blocks by the share of the chip that
 // they fill, 32 rows a CU: 64 and 128 heads up to 128 keys from a quarter (128 heads, 16 sequences of 96
@@ -284,8 +286,7 @@ int latent_chunk(const pa_cache* c, const pa_batch* b, const pa_attn* a, const H
 // 37.5 / 38.5), up to 384 nearly full (64 59.7 / 55.4; 32 48.6 / 51.8).  32 heads half fill a 64-row block
 // and still win there (64 sequences of 96 29.7 / 30.0, 32 24.5 / 28.2).
 bool latent_short(const pa_cache* c, const pa_batch* b, const pa_attn* a, int mq) {
-  const int64_t cap = (int64_t)b->max_blocks * c->block_size;
-  const int64_t keys = b->max_context_len > 0 ? std::min<int64_t>(b->max_context_len, cap) : cap;
+  const int64_t keys = (int64_t)b->max_blocks * c->block_size;
   const int64_t seq_rows = (int64_t)a->num_heads * mq;
   if (seq_rows < 32) return keys <= 96 || (keys <= 128 && b->batch >= 16);
   const int64_t rows = (int64_t)a->num_heads * b->num_tokens, full = 32 * (int64_t)device_cus();

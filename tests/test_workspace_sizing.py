@@ -206,6 +206,11 @@ def test_latent_blocks_follow_rows_and_keys(H, B, keys, wide):
     assert (n == SEGMENTS) == wide, n
 
 
+def test_latent_blocks_of_short_contexts_behind_a_long_table():
+    """The smaller blocks' grid covers the table: 16 heads, 4 contexts of 64 keys behind 8192."""
+    assert _latent([63] * 4, 16, table=8192) == SEGMENTS
+
+
 def test_latent_segments_are_asked_for_only_where_they_can_run():
     """The 64-row blocks read every row from the pages: without host metadata (operator) or
     PA_BATCH_NEW_ROWS_IN_CACHE (kernel entry), or with a slot mapping, they cannot run."""
