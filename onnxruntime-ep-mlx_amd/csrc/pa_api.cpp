@@ -629,8 +629,19 @@ struct SplitPlan {
 // 103.2, 16 of 2000 53.4 / 65.2 / 108.5 against 91.7 / 121.3 / 140.3; fp16, head 256, 8 of 2000 51.1 /
 // 82.5 / 122.4 against 60.6 / 123.0 / 137.2.  bf16 prompts at head 256 keep to the grid kernel below
 // 512 row blocks: 48 contexts of 1000 (197 MB) beside 1500 tokens 239.4 against 216.0, 32 of 2000
-// 230.7 against 257.9.
-int64_t split_min_bytes(const pa_cache* c, pa_dtype act) {
+// 230.7 against 257.9.  At heads 96 and 128 over 16-bit pages the bar is higher where the grid launch
+// takes a decode sequence for little more than a short prompt.  Prompts of one row block each
+// (one_block): from 800 Ki key rows on.  One of 30 tokens after 2000, bf16, 8 kv-heads of 128: 16
+// contexts of 3000 (156 MB) 71.5 / 52.9, 48 of 1000 75 / 70, 16 of 8000 (417 MB) 114 / 112, 48 of 3000
+// (469 MB) 123 / 141; head 96, 16 of 3000 (117 MB) 1.17 times as long split, 48 of 3000 (352 MB) 0.82
+// times.  (Head 64 0.5 .. 1.0, fp16 head 256 0.4 .. 1.04 and coded pages 0.2 .. 0.7 times at any size.)
+// Longer prompts in a batch whose row blocks leave workgroup slots free (few_blocks): from 192 Ki.  Split
+// takes, of whole, 4 kv-heads of 128, 16 contexts of 3000 or 48 of 1000 (160 Ki) beside 20 or 36 tokens
+// 1.09 .. 1.29; 8 kv-heads, 4 of 8000 (214 Ki) beside 36 .. 96 tokens 0.55 .. 0.90, 16 of 3000 (313 Ki)
+// 0.75 .. 0.87.
+int64_t split_min_bytes(const pa_cache* c, pa_dtype act, bool one_block, bool few_blocks) {
+  if ((one_block || few_blocks) && c->dtype == act && (c->head_dim == 96 || c->head_dim == 128))
+    return (int64_t)(one_block ? 800 : 192) * 1024 * c->head_dim * 4;
   return (int64_t)(act == PA_DTYPE_BFLOAT16 && c->head_dim > 128 ? 224 : 60) << 20;
 }
 
@@ -655,8 +666,10 @@ SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_
       keys += a->local_window_size > 0 ? std::min<int64_t>(ctx, (int64_t)a->local_window_size + nq) : ctx;
     }
   }
+  const int64_t blocks = ((int64_t)g * mq_long + pa::kPrefillRows - 1) / pa::kPrefillRows;
+  const bool few_blocks = blocks * b->batch * c->kv_heads < 2 * (int64_t)device_cus();
   if (n_long == 0 || n_long > pa::kMaxRanks || mq_short == 0 ||
-      keys * c->kv_heads * c->head_dim * 4 < split_min_bytes(c, act))
+      keys * c->kv_heads * c->head_dim * 4 < split_min_bytes(c, act, blocks == 1, few_blocks))
     return sp;
   sp.short_tokens = limit;
   sp.dec_batch = sp.pre_batch = *b;

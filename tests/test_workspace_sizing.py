@@ -225,3 +225,35 @@ def test_latent_segments_are_asked_for_only_where_they_can_run():
         n = lib.pa_attention_workspace_bytes_ex(C.byref(cache), C.byref(batch), C.byref(attn),
                                                 capi.PA_DTYPE_BFLOAT16, 0, 0)
         assert (n == SEGMENTS) == wide, (flags, n)
+
+
+# decode sequences and their contexts beside one prompt after 2000 keys; split / whole, us
+@pytest.mark.parametrize("kv,d,steps,past,nq,split", [
+    (8, 128, 16, 3000, 30, False),  # 71 / 53: a prompt of one row block
+    (8, 128, 48, 3000, 30, True),   # 123 / 141
+    (8, 128, 16, 3000, 40, True),   # two row blocks
+    (4, 128, 16, 3000, 40, False),  # 61 / 50: fewer key rows
+    (4, 128, 16, 8000, 40, True),
+    (8, 128, 4, 8000, 96, True),    # 54 / 73
+    (8, 96, 16, 3000, 30, False),
+    (8, 96, 48, 3000, 30, True),
+    (8, 128, 16, 400, 130, False),  # too few keys
+])
+def test_mixed_batches_split_by_the_keys_and_the_prompts_blocks(kv, d, steps, past, nq, split):
+    lib = capi.load()
+    cum = np.concatenate([np.arange(steps + 1), [steps + nq]]).astype(np.int32)
+    past = np.array([past] * steps + [2000], np.int32)
+    mb = -(-int((past + np.diff(cum)).max()) // 16)
+    dt = capi.PA_DTYPE_BFLOAT16
+    heads = 4 * kv
+    cache = capi.PaCache(FAKE, FAKE, None, None, (steps + 1) * mb, 16, kv, d, dt)
+    io = capi.PaIO(dt, int(cum[-1]), heads * d, FAKE, FAKE, FAKE, cache, FAKE, FAKE, FAKE, steps + 1, mb, None,
+                   None, 0, 0, None, None, None, None, cum.ctypes.data, past.ctypes.data, FAKE, None, FAKE,
+                   None, None, 0, 0)
+    node = capi.PaNode(heads, kv, 0.0, 0.0, -1, 0, 0, 0, 1, 1e-6)
+    n = [lib.pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io))]
+    io.host_cumulative_sequence_length = io.host_past_seqlens = None  # whole, on its plain plan
+    io.max_query_len = nq
+    n.append(lib.pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io)))
+    decode = kv * 16 * 128 * (d * 4 + 8)  # partials of the streaming decode's segments, at the least
+    assert (n[0] >= decode and n[0] > n[1]) == split, n
