@@ -189,10 +189,13 @@ int device_cus() {
 }
 
 // Per-sequence query and past lengths from host metadata (pa_paged_attention's host_* inputs),
-// when the caller gave them: they size the LATENT kernel's context chunks.
+// when the caller gave them: they size the LATENT kernel's context chunks and weigh the launches of
+// short prefills.  batch > 0: the arrays hold that many sequences, and the plan is for those of more
+// than longer_than new tokens (a batch split by query length).
 struct HostLens {
   const int32_t* cum = nullptr;
   const int32_t* past = nullptr;
+  int32_t batch = 0, longer_than = -1;
 };
 
 #ifndef PA_LATENT_PLAN
@@ -317,38 +320,71 @@ int64_t grid_chunk(int64_t units, int64_t slots, int ctx, int head_dim) {
   return std::min<int64_t>(std::max<int64_t>((ch + step - 1) / step * step, 256), INT32_MAX / 2);
 }
 
+// What the prefill launches of a batch have to do: its (row block, sequence, kv-head) items, the keys
+// that they see, the live keys of all kv-heads; from the host's lengths, or at the bounds without them.
+struct PrefillLoad {
+  double items = 0, seen = 0, rows = 0;
+};
+PrefillLoad prefill_load(const pa_cache* c, const pa_batch* b, int g, int64_t rbs, int64_t live,
+                         int64_t reach, const HostLens& hl) {
+  PrefillLoad l;
+  const int n = hl.batch > 0 ? hl.batch : b->batch;
+  for (int i = 0; hl.cum && hl.past && i < n; ++i) {
+    const int64_t nq = (int64_t)hl.cum[i + 1] - hl.cum[i];
+    if (nq <= 0 || nq <= hl.longer_than) continue;
+    const int64_t keys = std::min<int64_t>((int64_t)std::max(hl.past[i], 0) + nq, live);
+    const double blocks = (double)((g * nq + pa::kPrefillRows - 1) / pa::kPrefillRows);
+    l.items += blocks;
+    l.seen += blocks * (double)std::min(keys, reach);
+    l.rows += (double)keys;
+  }
+  if (l.items == 0) {
+    l.items = (double)b->batch * (double)rbs;
+    l.seen = l.items * (double)std::min(live, reach);
+    l.rows = (double)b->batch * (double)live;
+  }
+  l.items *= c->kv_heads;
+  l.seen *= c->kv_heads;
+  l.rows *= c->kv_heads;
+  return l;
+}
+
 // Whether a batch of fewer items than workgroup slots runs the planned image prefill all the same
 // (given the workspace): where the estimated time of its launches (images of every live key, the keys
-// that a slot walks when all share the work) is below the grid launch's (the keys of its chunks, cut
-// from the table's capacity, over its one or two workgroups a CU; the items' set-up; the partial rows
-// of every chunk).  seen: keys that a row block sees, fewer than the live ones under a window.
-// The figures (us, us a key and an item, head 256 apart) fit 6,880 calls timed both ways: fp16 and
+// that a slot walks when all share the work, the merge of items in parts) is below the grid launch's
+// (the keys of its chunks, cut from the table's capacity, over its one or two workgroups a CU; the
+// items' set-up; the partial rows of every chunk).  seen: keys that a row block sees at most, fewer
+// than the live ones under a window.
+// The figures (us, us a key and an item, by head size) fit 6,880 calls timed both ways: fp16 and
 // bf16, 1 .. 40 row blocks a sequence, 96 .. 500 items, pasts of 0 .. 3000 keys, windows, tables of 1, 2
-// and 8 times the context.  The choice is 0.75 % off the better of the two on average, 15 % at worst
+// and 8 times the context.  The choice is 0.5 % off the better of the two on average, 15 % at worst
 // against the grid (always planned: 430 %).  Planned / grid: bf16 32 heads of 128, 60 x 29 tokens
 // after 1000 197 / 141, 38 x 29 after 3000 in a window of 128 233 / 64; 2 x 512 after 1000 73 / 84, 2000
 // tokens 94 / 126; fp16 24 heads of 256, 10 x 253 after 3000 390 / 742; bf16 64 heads of 64, 2 x 253
-// after 1000 50 / 68.
+// after 1000 50 / 68.  The lengths of the sequences count, not the longest alone: 7 x 45 without a past
+// and one after 3000, bf16 32 heads of 128, 48 / 60, 30 x 29 62 / 73 (one after 1000 49 / 46).
 #ifndef PA_R2_UNITS
 #define PA_R2_UNITS 96
 #endif
 bool short_planned(int64_t units, int64_t slots, int ctx, int64_t live, int64_t seen,
-                   int64_t image_rows, int head_dim) {
+                   const PrefillLoad& l, int head_dim) {
   if (units < PA_R2_UNITS || live < 320) return false;
   const bool big = head_dim > 128;
   const double chunk = (double)grid_chunk(units, slots, ctx, head_dim);
   const double chunks = std::ceil((double)live / chunk);
   // workgroups with work a slot: between their mean and its round up
-  const double each = (double)units * std::max((double)seen / chunk, 1.0) / (double)(big ? slots / 2 : slots);
+  const double each = std::max(l.seen / chunk, l.items) / (double)(big ? slots / 2 : slots);
   const double grid_keys =
       std::min(chunk, (double)seen) * std::max(1.0, (each + std::ceil(each)) / 2);
-  const double plan_keys = std::max((double)units * (double)seen / (double)slots,
-                                    (double)std::min<int64_t>(seen, PA_FINE_MIN));
+  const double plan_keys =
+      std::max(l.seen / (double)slots, (double)std::min<int64_t>(seen, PA_FINE_MIN));
   const double rows = chunks > 1.0 ? chunks : 0.0;  // partial rows of an item, in items
   const double grid = (big ? 0.083 : 0.042) * grid_keys +
-                      (double)units * (big ? 0.08 + 0.055 * rows : 0.05 + 0.03 * rows);
-  const double plan = (big ? 0.11 : 0.042) * plan_keys + 1.8e-6 * (double)image_rows * head_dim +
-                      (head_dim == 128 ? 12.0 : 5.0);  // (beyond the grid launch's own start)
+                      l.items * (big ? 0.08 + 0.055 * rows : 0.05 + 0.03 * rows);
+  // beyond the grid launch's own start: the plan, and the merge where items come in parts
+  const bool parts = seen > PA_FINE_MIN;
+  const double more = big ? 0.0 : head_dim == 128 && parts ? 13.0 : head_dim == 64 && parts ? 7.0 : 4.0;
+  const double plan = (big ? 0.11 : 0.042) * plan_keys + 1.8e-6 * l.rows * head_dim + more;
   return plan < grid;
 }
 
@@ -457,7 +493,8 @@ Plan make_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype 
                        pa::prefill_mfma_supported(c->head_dim, act, c->dtype) &&
                        b->max_context_len > 0 &&
                        short_planned(units, target, ctx, live_keys, seen_keys,
-                                     (int64_t)b->batch * c->kv_heads * live_keys, c->head_dim) &&
+                                     prefill_load(c, b, g, rbs, live_keys, seen_keys, hl),
+                                     c->head_dim) &&
                        (int64_t)b->batch * c->kv_heads *
                                ((live_keys + pa::img_keys(c->head_dim) - 1) / pa::img_keys(c->head_dim)) *
                                pa::img_step_bytes(c->head_dim) <= kImgMaxBytes;
@@ -678,7 +715,8 @@ SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_
   sp.pre_batch.max_context_len = (int32_t)std::min<int64_t>(ctx_long, INT32_MAX);
   sp.pre_batch.batch = n_long;
   sp.dec = make_plan(c, &sp.dec_batch, a, act, 0, 0, false, 0, images);
-  sp.pre = make_plan(c, &sp.pre_batch, a, act, 0, 0, false, 0, images, false, HostLens(), true);
+  sp.pre = make_plan(c, &sp.pre_batch, a, act, 0, 0, false, 0, images, false,
+                     HostLens{hl.cum, hl.past, b->batch, limit}, true);
   if (!sp.dec.balanced || sp.pre.kind != 2 || sp.pre.sub_batch > 0) return sp;
   sp.seq_off = workspace_for(c, &sp.pre_batch, a, sp.pre);
   sp.bytes = std::max(workspace_for(c, &sp.dec_batch, a, sp.dec),

@@ -136,6 +136,7 @@ def test_short_prefills_plan_images_of_a_bounded_context_only():
     (32, 8, 128, 2, 512, 1000, -1, 0, True),    # 73 / 84
     (32, 8, 128, 1, 2000, 4000, 128, 0, True),  # 52 / 86: a window over many row blocks
     (64, 8, 64, 8, 45, 1000, -1, 0, True),      # 45 / 65
+    (32, 8, 128, 3, 125, 3000, 128, 0, True),   # 45 / 48: each item sees its window alone
     (32, 8, 128, 4, 125, 1000, -1, 8960, True),  # 55 / 69: chunks cut from a table of 8 contexts
 ])
 def test_short_prefills_weigh_images_against_what_reads_them(H, KV, d, B, nq, past, window, table,
@@ -148,6 +149,19 @@ def test_short_prefills_weigh_images_against_what_reads_them(H, KV, d, B, nq, pa
                                     H=H, d=d, host=host, cache=act, act=act, window=window)
             n.append(lib.pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io)))
         assert (n[0] != n[1]) == planned
+
+
+@pytest.mark.parametrize("past,planned", [(0, False), (3000, True)])  # 48 / 60 us planned / grid
+def test_short_prefills_weigh_the_batch_by_its_sequences(past, planned):
+    """7 prompts of 45 tokens without a past and one with: the grid launch cuts every sequence into
+    chunks of the longest context's table, the images hold what is there."""
+    lib = capi.load()
+    n = []
+    for host in (True, False):
+        node, io, keep = _paged([0] * 7 + [past], 45, -(-(past + 45) // 16), H=32, host=host,
+                                cache=capi.PA_DTYPE_BFLOAT16)
+        n.append(lib.pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io)))
+    assert (n[0] != n[1]) == planned
 
 
 def test_forced_prefill_kind_splits_short_batches_over_the_grid():
