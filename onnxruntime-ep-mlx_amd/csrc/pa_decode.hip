@@ -1195,15 +1195,21 @@ decode_balanced_kernel(const AttnParams p) {
 // A device-scope fence per piece inside the decode kernel (to let the last piece merge) writes
 // back the XCD's L2 and measured far slower than this separate launch.
 constexpr int kMergeDepth = 4;
-// Head dims of a workgroup's slice: 64 (16 lanes per partial), 32 at head 96; the one-wavefront
-// workgroups of batches with few partials per sequence take up to 256, for fewer workgroups.
+// Head dims of a workgroup's slice SL: 64 (16 lanes per partial), 32 at head 96; the one-wavefront
+// workgroups of batches with few partials per sequence take up to 256, for fewer workgroups.  At head
+// 96 those take the whole row only where the slices come to more than kMergeMany (24 a CU), which then
+// queue: 24 heads over 8, 64 sequences of two tokens (36 a CU) after 150 .. 300 the call 28.8 us
+// against 33.6 with three slices, after 500 .. 1000 51.2 / 56.4.  Below, the 32 partials that a slice
+// has in flight against the whole row's 8 count for more where one sequence is long: 32 sequences of
+// two tokens (18 a CU) after 60, one of them after 16000, 42.0 / 34.6.
+constexpr int64_t kMergeMany = 24 * 256;
 template <int D, int NT>
 constexpr int merge_slice() {
   return D % 64 != 0 ? 32 : NT > 64 ? 64 : D;
 }
-template <typename TT, int D, int NT>
+template <typename TT, int D, int NT, int SL>
 __global__ __launch_bounds__(NT) void balanced_merge_kernel(const AttnParams p) {
-  constexpr int SL = merge_slice<D, NT>(), LP = SL / 4, PG = NT / LP, NW = NT / 64;
+  constexpr int LP = SL == 96 ? 32 : SL / 4, PG = NT / LP, NW = NT / 64;
   const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int kh = blockIdx.x % p.kv_heads, rest = blockIdx.x / p.kv_heads;
   const int slice = rest % (D / SL), r = rest / (D / SL);
@@ -1230,7 +1236,8 @@ __global__ __launch_bounds__(NT) void balanced_merge_kernel(const AttnParams p) 
   const int nparts = (int)((Pb + nb - 1) / seg_l) - f + 1;
   if (nparts <= 1) return;  // written directly by the decode kernel
 
-  const int grp = tid / LP, d0 = slice * SL + 4 * (tid % LP);
+  // (a slice of 96: lanes 24 .. 31 of a group read its last 16 bytes again and write nothing)
+  const int grp = tid / LP, d0 = slice * SL + 4 * min(tid % LP, SL / 4 - 1);
   const int64_t row0 = (((int64_t)f + b) * p.kv_heads + kh) * 16 + r;
   const int64_t pitch = (int64_t)p.kv_heads * 16;  // rows between consecutive partials
   float M = kNegInf, lsum = 0.0f;
@@ -1285,7 +1292,7 @@ __global__ __launch_bounds__(NT) void balanced_merge_kernel(const AttnParams p) 
     if (tid >= LP) return;
 #pragma unroll
     for (int w = 1; w < NW; ++w) meet(wml[w].x, wml[w].y, wacc[w][tid]);
-  } else if (tid >= LP) {
+  } else if (tid >= SL / 4) {
     return;
   }
   const int h = kh * g + r % g;
@@ -1413,11 +1420,15 @@ hipError_t launch_decode_mfma(const AttnParams& p, pa_dtype act, pa_dtype cache_
 // 32-key step of its window or block table: 64 hold 4 groups of 4 partials in flight, 256 four times
 // and 1024 sixteen times as many, all of an average row in one round trip; more threads than that
 // only wait on each other.
-template <typename TT, int D, int NT>
+template <typename TT, int D, int NT, int SL = merge_slice<D, NT>()>
 void launch_merge_nt(const AttnParams& p, hipStream_t s) {
   const int rows = std::min(16, (p.num_heads / p.kv_heads) * std::max(p.max_query_len, 1));
-  const dim3 grid(p.kv_heads * (D / merge_slice<D, NT>()) * rows, p.batch);
-  hipLaunchKernelGGL((balanced_merge_kernel<TT, D, NT>), grid, dim3(NT), 0, s, p);
+  const dim3 grid(p.kv_heads * (D / SL) * rows, p.batch);
+  if constexpr (NT == 64 && SL < D) {
+    if ((int64_t)grid.x * grid.y > kMergeMany)
+      return launch_merge_nt<TT, D, NT, D>(p, s);
+  }
+  hipLaunchKernelGGL((balanced_merge_kernel<TT, D, NT, SL>), grid, dim3(NT), 0, s, p);
 }
 template <typename TT, int D>
 void launch_merge_d(const AttnParams& p, hipStream_t s) {

@@ -16,6 +16,7 @@ MERGES = [
     (8, 2, 256, 256, [16383]), (16, 1, 128, 16, [4097, 0, 31, 20000]),
     (8, 2, 128, 16, [500] * 11 + [7000]), (8, 4, 64, 16, [9 * i for i in range(70)]),
     (2, 2, 96, 16, [63, 64, 65, 2000] * 5),
+    (64, 8, 96, 16, [40 * i for i in range(39)] + [6000]),  # many workgroups: whole rows of 96
 ]
 
 
