@@ -210,7 +210,7 @@ size_t pa_attention_workspace_bytes_ex(const pa_cache* cache, const pa_batch* ba
  *     or 512 dims (MLA 576 / 512): its matrix-core kernels, all heads served by one read of each
  *     row per 16 or 32 grouped query rows, and per 64 at 576 / 512 with 16 or more of them, the new
  *     rows in the pages, whole 16-row tiles per page and the queried workspace, but for short contexts
- *     that the smaller blocks take in one round;
+ *     behind short tables that the smaller blocks take in one round;
  *   - fp32 activations, other head sizes, other LATENT shapes and forced split-K chunks over
  *     byte-coded pages: the VALU kernel.
  * batch->max_query_len = 0 is read as num_tokens. */
