@@ -1315,7 +1315,12 @@ __device__ __forceinline__ void img_load(const AttnParams& p, int id, ImgGroup<N
   constexpr int SPW = NT / 256, KEYS = img_keys(D), PCS = ImgGroup<NT, D>::PCS;
   constexpr int CH = ImgGroup<NT, D>::CH;
   const int nj = (p.img_steps + SPW - 1) / SPW;
-  const int jb = id % nj, kh = (id / nj) % p.kv_heads, rank = min(id / (nj * p.kv_heads), p.seqs - 1);
+  // Workgroups go round-robin to the 8 XCDs.  With an even number of groups a row, the first ones,
+  // which alone have keys in a short sequence, would all be on one or a few: 48 decode sequences of
+  // 200 .. 300 keys beside one of 2030, 8 kv-heads of 128, took 93 us for the images.  Each row then
+  // starts one group later; odd numbers spread them by themselves.
+  const int row = id / nj, jb = (nj & 1) ? id % nj : (id + row) % nj;
+  const int kh = row % p.kv_heads, rank = min(row / p.kv_heads, p.seqs - 1);
   const int bn = seq_of_rank(p, __builtin_amdgcn_readfirstlane(rank)), b = max(bn, 0);
   const int s0 = min(max(p.cum[b], 0), p.num_tokens);
   const int s1 = bn < 0 ? s0 : min(max(p.cum[b + 1], s0), p.num_tokens);
