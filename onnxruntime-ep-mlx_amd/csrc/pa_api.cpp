@@ -658,7 +658,7 @@ struct SplitPlan {
   size_t seq_off = 0, bytes = 0;  // list of the prefill sequences, workspace in all
 };
 
-// Key/value bytes (as 16-bit rows) of the decode sequences from which a batch is split.  The split
+// Whether a batch is split: from how many key/value bytes (as 16-bit rows) of the decode sequences on.  The split
 // costs the decode's two launches, and few long rows lose the planned launch that all rows together
 // fill; what it saves grows with the decode sequences' contexts.  One prompt of 64 / 300 / 1500 tokens
 // beside them, bf16, 8 kv-heads of 128, split against whole: 16 contexts of 500 (33 MB) 37.6 / 59.3 /
@@ -676,10 +676,16 @@ struct SplitPlan {
 // takes, of whole, 4 kv-heads of 128, 16 contexts of 3000 or 48 of 1000 (160 Ki) beside 20 or 36 tokens
 // 1.09 .. 1.29; 8 kv-heads, 4 of 8000 (214 Ki) beside 36 .. 96 tokens 0.55 .. 0.90, 16 of 3000 (313 Ki)
 // 0.75 .. 0.87.
-int64_t split_min_bytes(const pa_cache* c, pa_dtype act, bool one_block, bool few_blocks) {
-  if ((one_block || few_blocks) && c->dtype == act && (c->head_dim == 96 || c->head_dim == 128))
-    return (int64_t)(one_block ? 800 : 192) * 1024 * c->head_dim * 4;
-  return (int64_t)(act == PA_DTYPE_BFLOAT16 && c->head_dim > 128 ? 224 : 60) << 20;
+// These bars count the whole contexts, which the grid launch's chunks span, the bytes only the keys in a
+// window: in a window of 1024, 8 kv-heads of 128 beside 30 tokens, 16 contexts of 3000 take 1.27 times as
+// long split, 16 of 8000 45 us against 54, 48 of 3000 69 against 75.
+bool split_pays(const pa_cache* c, pa_dtype act, int64_t keys, int64_t contexts, bool one_block,
+                bool few_blocks) {
+  if ((one_block || few_blocks) && c->dtype == act && (c->head_dim == 96 || c->head_dim == 128) &&
+      contexts * c->kv_heads < (one_block ? 800 : 192) * 1024)
+    return false;
+  return keys * c->kv_heads * c->head_dim * 4 >=
+         (int64_t)(act == PA_DTYPE_BFLOAT16 && c->head_dim > 128 ? 224 : 60) << 20;
 }
 
 SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_dtype act,
@@ -690,7 +696,7 @@ SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_
   if (g < 1 || g > 16) return sp;
   const int limit = 16 / g;
   int n_long = 0, mq_short = 0, mq_long = 0;
-  int64_t keys = 0, ctx_long = 0;
+  int64_t keys = 0, contexts = 0, ctx_long = 0;  // keys: of the decode sequences' contexts, those in a window
   for (int i = 0; i < b->batch; ++i) {
     const int nq = hl.cum[i + 1] - hl.cum[i];
     const int64_t ctx = (int64_t)std::max(hl.past[i], 0) + nq;
@@ -700,13 +706,14 @@ SplitPlan split_plan(const pa_cache* c, const pa_batch* b, const pa_attn* a, pa_
       ctx_long = std::max(ctx_long, ctx);
     } else if (nq > 0) {
       mq_short = std::max(mq_short, nq);
+      contexts += ctx;
       keys += a->local_window_size > 0 ? std::min<int64_t>(ctx, (int64_t)a->local_window_size + nq) : ctx;
     }
   }
   const int64_t blocks = ((int64_t)g * mq_long + pa::kPrefillRows - 1) / pa::kPrefillRows;
   const bool few_blocks = blocks * b->batch * c->kv_heads < 2 * (int64_t)device_cus();
   if (n_long == 0 || n_long > pa::kMaxRanks || mq_short == 0 ||
-      keys * c->kv_heads * c->head_dim * 4 < split_min_bytes(c, act, blocks == 1, few_blocks))
+      !split_pays(c, act, keys, contexts, blocks == 1, few_blocks))
     return sp;
   sp.short_tokens = limit;
   sp.dec_batch = sp.pre_batch = *b;

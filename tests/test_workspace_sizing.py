@@ -242,18 +242,20 @@ def test_latent_segments_are_asked_for_only_where_they_can_run():
 
 
 # decode sequences and their contexts beside one prompt after 2000 keys; split / whole, us
-@pytest.mark.parametrize("kv,d,steps,past,nq,split", [
-    (8, 128, 16, 3000, 30, False),  # 71 / 53: a prompt of one row block
-    (8, 128, 48, 3000, 30, True),   # 123 / 141
-    (8, 128, 16, 3000, 40, True),   # two row blocks
-    (4, 128, 16, 3000, 40, False),  # 61 / 50: fewer key rows
-    (4, 128, 16, 8000, 40, True),
-    (8, 128, 4, 8000, 96, True),    # 54 / 73
-    (8, 96, 16, 3000, 30, False),
-    (8, 96, 48, 3000, 30, True),
-    (8, 128, 16, 400, 130, False),  # too few keys
+@pytest.mark.parametrize("kv,d,steps,past,nq,window,split", [
+    (8, 128, 16, 3000, 30, -1, False),  # 71 / 53: a prompt of one row block
+    (8, 128, 48, 3000, 30, -1, True),   # 123 / 141
+    (8, 128, 16, 3000, 40, -1, True),   # two row blocks
+    (4, 128, 16, 3000, 40, -1, False),  # 61 / 50: fewer key rows
+    (4, 128, 16, 8000, 40, -1, True),
+    (8, 128, 4, 8000, 96, -1, True),    # 54 / 73
+    (8, 96, 16, 3000, 30, -1, False),
+    (8, 96, 48, 3000, 30, -1, True),
+    (8, 128, 16, 400, 130, -1, False),  # too few keys
+    (8, 128, 16, 3000, 30, 1024, False),  # the whole contexts count
+    (8, 128, 16, 8000, 30, 1024, True),   # 45 / 54
 ])
-def test_mixed_batches_split_by_the_keys_and_the_prompts_blocks(kv, d, steps, past, nq, split):
+def test_mixed_batches_split_by_the_keys_and_the_prompts_blocks(kv, d, steps, past, nq, window, split):
     lib = capi.load()
     cum = np.concatenate([np.arange(steps + 1), [steps + nq]]).astype(np.int32)
     past = np.array([past] * steps + [2000], np.int32)
@@ -264,7 +266,7 @@ def test_mixed_batches_split_by_the_keys_and_the_prompts_blocks(kv, d, steps, pa
     io = capi.PaIO(dt, int(cum[-1]), heads * d, FAKE, FAKE, FAKE, cache, FAKE, FAKE, FAKE, steps + 1, mb, None,
                    None, 0, 0, None, None, None, None, cum.ctypes.data, past.ctypes.data, FAKE, None, FAKE,
                    None, None, 0, 0)
-    node = capi.PaNode(heads, kv, 0.0, 0.0, -1, 0, 0, 0, 1, 1e-6)
+    node = capi.PaNode(heads, kv, 0.0, 0.0, window, 0, 0, 0, 1, 1e-6)
     n = [lib.pa_paged_attention_workspace_bytes(C.byref(node), C.byref(io))]
     io.host_cumulative_sequence_length = io.host_past_seqlens = None  # whole, on its plain plan
     io.max_query_len = nq
