@@ -1557,10 +1557,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void pr
   constexpr int NB = 1024;  // buckets of 32-key steps (the last one holds everything longer)
   __shared__ int hist[NB];
   __shared__ unsigned long long total_keys;
-  __shared__ int nslots;  // fp32 partial slots given out (plan_fine)
+  __shared__ int nslots;         // plan_fine: fp32 partial slots given out,
+  __shared__ int nlong, longest;  // items of more than PA_FINE_MIN keys, keys of the longest
   const int tid = threadIdx.x;
   for (int i = tid; i < NB; i += NT) hist[i] = 0;
-  if (tid == 0) total_keys = 0, nslots = 0;
+  if (tid == 0) total_keys = 0, nslots = 0, nlong = 0, longest = 0;
   // A batch split by query length: the sequences of the prefill ranks, for this kernel and, as
   // plan_seq, for the launches behind it (one wavefront, in batch order).
   __shared__ int seqs[kMaxRanks];
@@ -1602,6 +1603,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void pr
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) mine += __shfl_xor(mine, o, 64);
   if ((tid & 63) == 0) atomicAdd(&total_keys, mine);
+  if (p.plan_fine) {  // fewer items than workgroup slots: the cached ones are all
+    int len = 0;
+#pragma unroll
+    for (int j = 0; j < kCached; ++j) {
+      const int n = cached[j].end >= 0 ? cached[j].end - cached[j].first : 0;
+      const uint64_t m = __ballot(n > PA_FINE_MIN);
+      if ((tid & 63) == 0 && m) atomicAdd(&nlong, __builtin_popcountll(m));
+      len = max(len, n);
+    }
+    for (int o = 1; o < 64; o <<= 1) len = max(len, __shfl_xor(len, o, 64));
+    if ((tid & 63) == 0 && len > 0) atomicMax(&longest, len);
+  }
   __syncthreads();
   const long long thr = max((long long)PA_PLAN_SPLIT_MIN,
                            (long long)(total_keys * PA_PLAN_SPLIT_PCT / 100) / max(p.plan_slots, 1));
@@ -1622,8 +1635,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void pr
   // us a call; 320 items of 48 steps 184 / 184 / 172 / 173; 256 items at head 256 248 / 218 / 264 /
   // 227: 175 % splits the first in three and the last in two, and leaves the second whole.
   const bool fine = p.plan_fine && total_keys < (unsigned long long)PA_PLAN_SPLIT_MIN * p.plan_slots;
-  const int even = max(PA_FINE_MIN, (int)min(total_keys * kFinePct / (100ull * max(p.plan_slots, 1)),
-                                             (unsigned long long)INT32_MAX / 2));
+  const int even = __builtin_amdgcn_readfirstlane(
+      longest <= fine_whole(nlong, IMGD)
+          ? INT32_MAX / 2
+          : max(PA_FINE_MIN, (int)min(total_keys * kFinePct / (100ull * max(p.plan_slots, 1)),
+                                      (unsigned long long)INT32_MAX / 2)));
   auto steps_of = [&](const ItemKeys& k) { return (k.end - k.first + step - 1) / step; };
   auto part_steps = [&](const ItemKeys& k) {  // key steps of each of the item's parts
     const int s = steps_of(k), n = min((k.end - k.first + even - 1) / even, kFineParts);
