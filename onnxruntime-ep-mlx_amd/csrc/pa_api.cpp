@@ -320,30 +320,42 @@ int64_t grid_chunk(int64_t units, int64_t slots, int ctx, int head_dim) {
   return std::min<int64_t>(std::max<int64_t>((ch + step - 1) / step * step, 256), INT32_MAX / 2);
 }
 
-// What the prefill launches of a batch have to do: its (row block, sequence, kv-head) items, the keys
-// that they see, the live keys of all kv-heads; from the host's lengths, or at the bounds without them.
+// What the prefill launches of a batch have to do: its (row block, sequence, kv-head) items, their query
+// rows in whole blocks, the items that may be split, the keys that they see, the live keys of all
+// kv-heads, the image workgroups that find none; from the host's lengths, or at the bounds without them.
 struct PrefillLoad {
-  double items = 0, seen = 0, rows = 0;
+  double items = 0, blocks = 0, longer = 0, seen = 0, rows = 0, empty = 0;
 };
 PrefillLoad prefill_load(const pa_cache* c, const pa_batch* b, int g, int64_t rbs, int64_t live,
                          int64_t reach, const HostLens& hl) {
   PrefillLoad l;
   const int n = hl.batch > 0 ? hl.batch : b->batch;
+  const int64_t group = 4 * pa::img_keys(c->head_dim);  // keys of an image workgroup
+  const double groups = (double)b->batch * (double)((live + group - 1) / group);
+  l.empty = groups;
   for (int i = 0; hl.cum && hl.past && i < n; ++i) {
     const int64_t nq = (int64_t)hl.cum[i + 1] - hl.cum[i];
     if (nq <= 0 || nq <= hl.longer_than) continue;
     const int64_t keys = std::min<int64_t>((int64_t)std::max(hl.past[i], 0) + nq, live);
     const double blocks = (double)((g * nq + pa::kPrefillRows - 1) / pa::kPrefillRows);
     l.items += blocks;
+    l.blocks += (double)(g * nq) / pa::kPrefillRows;
+    l.empty -= (double)((keys + group - 1) / group);
+    if (std::min(keys, reach) > PA_FINE_MIN) l.longer += blocks;
     l.seen += blocks * (double)std::min(keys, reach);
     l.rows += (double)keys;
   }
   if (l.items == 0) {
-    l.items = (double)b->batch * (double)rbs;
+    l.items = l.blocks = (double)b->batch * (double)rbs;
+    l.empty = 0.0;
+    l.longer = std::min(live, reach) > PA_FINE_MIN ? l.items : 0.0;
     l.seen = l.items * (double)std::min(live, reach);
     l.rows = (double)b->batch * (double)live;
   }
   l.items *= c->kv_heads;
+  l.blocks *= c->kv_heads;
+  l.empty *= c->kv_heads;
+  l.longer *= c->kv_heads;
   l.seen *= c->kv_heads;
   l.rows *= c->kv_heads;
   return l;
@@ -353,16 +365,18 @@ PrefillLoad prefill_load(const pa_cache* c, const pa_batch* b, int g, int64_t rb
 // (given the workspace): where the estimated time of its launches (images of every live key, the keys
 // that a slot walks when all share the work, the merge of items in parts) is below the grid launch's
 // (the keys of its chunks, cut from the table's capacity, over its one or two workgroups a CU; the
-// items' set-up; the partial rows of every chunk).  seen: keys that a row block sees at most, fewer
-// than the live ones under a window.
-// The figures (us, us a key and an item, by head size) fit 6,880 calls timed both ways: fp16 and
-// bf16, 1 .. 40 row blocks a sequence, 96 .. 500 items, pasts of 0 .. 3000 keys, windows, tables of 1, 2
-// and 8 times the context.  The choice is 0.5 % off the better of the two on average, 15 % at worst
-// against the grid (always planned: 430 %).  Planned / grid: bf16 32 heads of 128, 60 x 29 tokens
-// after 1000 197 / 141, 38 x 29 after 3000 in a window of 128 233 / 64; 2 x 512 after 1000 73 / 84, 2000
-// tokens 94 / 126; fp16 24 heads of 256, 10 x 253 after 3000 390 / 742; bf16 64 heads of 64, 2 x 253
-// after 1000 50 / 68.  The lengths of the sequences count, not the longest alone: 7 x 45 without a past
-// and one after 3000, bf16 32 heads of 128, 48 / 60, 30 x 29 62 / 73 (one after 1000 49 / 46).
+// rows read and written; the partial rows of every chunk).  seen: keys that a row block sees at most,
+// fewer than the live ones under a window.
+// The figures (us, us a key, a row block and an empty image workgroup, by head size) fit 7,690 calls
+// timed both ways: fp16 and bf16, 1 .. 40 row blocks a sequence, 96 .. 500 items, pasts of 0 .. 3000
+// keys, windows, tables of 1, 2 and 8 times the context, one long context among short ones, decode
+// sequences beside prompts.  The choice is 0.4 % off the better of the two on average; against the grid
+// it loses 14 % at worst without decode sequences and 23 % with them (always planned: 430 %).  Planned /
+// grid: bf16 32 heads of 128, 60 x 29 tokens after 1000 197 / 141, 38 x 29 after 3000 in a window of 128
+// 233 / 64; 2 x 512 after 1000 73 / 84, 2000 tokens 94 / 126; fp16 24 heads of 256, 10 x 253 after 3000
+// 390 / 742; bf16 64 heads of 64, 2 x 253 after 1000 50 / 68.  The lengths of the sequences count, not the
+// longest alone: 7 x 45 without a past and one after 3000, bf16 32 heads of 128, 48 / 60, 30 x 29 62 / 73;
+// 48 decode sequences of 200 .. 300 keys beside 30 tokens after 2000 86 / 64.
 #ifndef PA_R2_UNITS
 #define PA_R2_UNITS 96
 #endif
@@ -376,15 +390,18 @@ bool short_planned(int64_t units, int64_t slots, int ctx, int64_t live, int64_t 
   const double each = std::max(l.seen / chunk, l.items) / (double)(big ? slots / 2 : slots);
   const double grid_keys =
       std::min(chunk, (double)seen) * std::max(1.0, (each + std::ceil(each)) / 2);
-  const double plan_keys =
-      std::max(l.seen / (double)slots, (double)std::min<int64_t>(seen, PA_FINE_MIN));
-  const double rows = chunks > 1.0 ? chunks : 0.0;  // partial rows of an item, in items
+  const double rows = chunks > 1.0 ? chunks : 0.0;  // partial rows, in rows
   const double grid = (big ? 0.083 : 0.042) * grid_keys +
-                      l.items * (big ? 0.08 + 0.055 * rows : 0.05 + 0.03 * rows);
-  // beyond the grid launch's own start: the plan, and the merge where items come in parts
-  const bool parts = seen > PA_FINE_MIN;
-  const double more = big ? 0.0 : head_dim == 128 && parts ? 13.0 : head_dim == 64 && parts ? 7.0 : 4.0;
-  const double plan = (big ? 0.11 : 0.042) * plan_keys + 1.8e-6 * l.rows * head_dim + more;
+                      l.blocks * (big ? 0.08 + 0.055 * rows : 0.05 + 0.03 * rows);
+  // in parts, or whole: the keys of a slot, and what comes beyond the grid launch's own start
+  const bool parts = seen > pa::fine_whole((int)l.longer, head_dim);
+  const double slot_keys = l.seen / (double)slots;
+  const double walk = big     ? 0.05 * slot_keys
+                      : parts ? 0.024 * std::max(slot_keys, (double)PA_FINE_MIN)
+                              : 0.04 * slot_keys;
+  const double more = parts ? (big ? 21.0 : head_dim == 128 ? 17.0 : head_dim == 96 ? 8.0 : 3.0)
+                            : (big ? 8.0 : head_dim == 128 ? 11.0 : head_dim == 96 ? 6.0 : 8.0);
+  const double plan = walk + 1.8e-6 * l.rows * head_dim + 0.006 * l.empty + more;
   return plan < grid;
 }
 

@@ -136,7 +136,7 @@ def test_short_prefills_plan_images_of_a_bounded_context_only():
     (32, 8, 128, 2, 512, 1000, -1, 0, True),    # 73 / 84
     (32, 8, 128, 1, 2000, 4000, 128, 0, True),  # 52 / 86: a window over many row blocks
     (64, 8, 64, 8, 45, 1000, -1, 0, True),      # 45 / 65
-    (32, 8, 128, 3, 125, 3000, 128, 0, True),   # 45 / 48: each item sees its window alone
+    (32, 8, 128, 6, 125, 1000, 128, 0, True),   # 42 / 62: few keys an item, no parts
     (32, 8, 128, 4, 125, 1000, -1, 8960, True),  # 55 / 69: chunks cut from a table of 8 contexts
 ])
 def test_short_prefills_weigh_images_against_what_reads_them(H, KV, d, B, nq, past, window, table,
@@ -252,6 +252,7 @@ def test_latent_segments_are_asked_for_only_where_they_can_run():
     (8, 96, 16, 3000, 30, -1, False),
     (8, 96, 48, 3000, 30, -1, True),
     (8, 128, 16, 400, 130, -1, False),  # too few keys
+    (8, 128, 48, 300, 30, -1, False),   # nor over images, most of whose workgroups find no keys: 86 / 64
     (8, 128, 16, 3000, 30, 1024, False),  # the whole contexts count
     (8, 128, 16, 8000, 30, 1024, True),   # 45 / 54
 ])
