@@ -412,13 +412,15 @@ static_assert(kFinePct >= 100, "plan_cap counts one slot per even share");
 #endif
 // No item of a short planned prefill is split while the longest has at most this many keys, `items`
 // being those of more than PA_FINE_MIN: what the parts save grows with the longest walk, what they
-// write and merge with the number of items (128 rows of fp32 each, twice).  Whole / in parts, us a call:
-// 8 kv-heads of 64 over fp8 pages, 12 prompts of 48 tokens after 393 keys (288 items) 34 / 39; 4 of 128,
-// 5 of 48 after 393 (60) 35.8 / 37.5, after 600 40 / 40; 2 of 100 .. 200 after 1000 (56) 56 / 43.  The line
-// fits 1,500 calls over 16-bit and coded pages, 96 .. 500 and 8 .. 500 items; it is within 0.7 % of the better
-// choice on average (parts from PA_FINE_MIN on: 2 .. 10 %).
+// write and merge with the number of items (128 rows of fp32 each, twice); at head 256 little up to 128
+// items, which leave half of the CUs without one.  Whole / in parts, us a call: 8 kv-heads of 64 over
+// fp8 pages, 12 prompts of 48 tokens after 393 keys (288 items) 34 / 39; 4 of 128, 5 of 48 after 393 (60)
+// 35.8 / 37.5, after 600 40 / 40; 2 of 100 .. 200 after 1000 (56) 56 / 43.  The lines fit 2,300 calls over
+// 16-bit and coded pages, 96 .. 500 and 8 .. 500 items, within 0.2 .. 1.1 % of the better choice on
+// average by page and head (in parts from PA_FINE_MIN on: 1.3 .. 7 %), 13 % at worst.
 __host__ __device__ constexpr int fine_whole(int items, int head_dim) {
-  return head_dim > 128 ? 350 + items * 3 / 2 : 350 + items * 4 < 1024 ? 350 + items * 4 : 1024;
+  const int keys = head_dim > 128 ? 4 * items - 100 : 4 * items + 350;
+  return keys < 350 ? 350 : keys > 1024 ? 1024 : keys;
 }
 // Split threshold of long planned prefills, in keys, at least (see prefill_plan_kernel).
 #ifndef PA_PLAN_SPLIT_MIN

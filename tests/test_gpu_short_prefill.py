@@ -17,9 +17,9 @@ SHAPES = [
     (64, 8, 64, 256, [511], [0]), (8, 4, 96, 16, [2000, 700], [100, 2500]),
     (24, 4, 256, 16, [513], [700]), (24, 4, 256, 32, [100, 90, 110, 200], [3000, 0, 500, 129]),
     (32, 8, 128, 16, [500], [0]), (64, 8, 64, 16, [177], [143]), (64, 8, 64, 16, [176], [144]),
-    # the longest item at the most keys that stay whole, and one more: 96 items of 734, 128 of 542
+    # the longest item at the most keys that stay whole, and one more: 96 items of 734, 128 of 412
     (64, 8, 64, 16, [177], [557]), (64, 8, 64, 16, [177], [558]),
-    (24, 4, 256, 16, [150] * 4, [392] * 4), (24, 4, 256, 16, [150] * 4, [393, 0, 10, 392]),
+    (24, 4, 256, 16, [150] * 4, [262] * 4), (24, 4, 256, 16, [150] * 4, [263, 262, 150, 262]),
 ]
 FORMS = [dict(rot=32), dict(dtype="float16", rot=32),
          dict(dtype="float16", window=700, softcap=20.0, sink=True), dict(window=130, sink=True)]
