@@ -1315,11 +1315,16 @@ __device__ __forceinline__ void img_load(const AttnParams& p, int id, ImgGroup<N
   constexpr int SPW = NT / 256, KEYS = img_keys(D), PCS = ImgGroup<NT, D>::PCS;
   constexpr int CH = ImgGroup<NT, D>::CH;
   const int nj = (p.img_steps + SPW - 1) / SPW;
-  // Workgroups go round-robin to the 8 XCDs.  With an even number of groups a row, the first ones,
-  // which alone have keys in a short sequence, would all be on one or a few: 48 decode sequences of
-  // 200 .. 300 keys beside one of 2030, 8 kv-heads of 128, took 93 us for the images.  Each row then
-  // starts one group later; odd numbers spread them by themselves.
-  const int row = id / nj, jb = (nj & 1) ? id % nj : (id + row) % nj;
+  // Workgroups go round-robin to the 8 XCDs.  With a multiple of 8 groups a row, the first ones, which
+  // alone have keys in a short sequence, would all be on one (few with other even numbers): 48 decode
+  // sequences of 200 .. 300 keys beside one of 2030, 8 kv-heads of 128, took 93 us for the images.  Rows
+  // of 8 groups or more therefore start at one of eight; odd numbers spread them by themselves.
+  const int row = id / nj;
+  int jb = id - row * nj;
+  if (nj >= 8 && !(nj & 1)) {
+    jb += row & 7;
+    if (jb >= nj) jb -= nj;
+  }
   const int kh = row % p.kv_heads, rank = min(row / p.kv_heads, p.seqs - 1);
   const int bn = seq_of_rank(p, __builtin_amdgcn_readfirstlane(rank)), b = max(bn, 0);
   const int s0 = min(max(p.cum[b], 0), p.num_tokens);
