@@ -418,9 +418,11 @@ static_assert(kFinePct >= 100, "plan_cap counts one slot per even share");
 // 35.8 / 37.5, after 600 40 / 40; 2 of 100 .. 200 after 1000 (56) 56 / 43.  The lines fit 2,300 calls over
 // 16-bit and coded pages, 96 .. 500 and 8 .. 500 items, within 0.2 .. 1.1 % of the better choice on
 // average by page and head (in parts from PA_FINE_MIN on: 1.3 .. 7 %), 13 % at worst.
+// Many items of uneven length end nearer 1000 keys: head 256, two prompts of 1006 tokens 104.4 / 101.8.
 __host__ __device__ constexpr int fine_whole(int items, int head_dim) {
   const int keys = head_dim > 128 ? 4 * items - 100 : 4 * items + 350;
-  return keys < 350 ? 350 : keys > 1024 ? 1024 : keys;
+  const int most = head_dim > 128 ? 950 : 1024;
+  return keys < 350 ? 350 : keys > most ? most : keys;
 }
 // Split threshold of long planned prefills, in keys, at least (see prefill_plan_kernel).
 #ifndef PA_PLAN_SPLIT_MIN
